@@ -21,7 +21,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libkmoe.so")
-SOURCES = ["api.hip", "route.hip", "expert.hip", "weights.hip", "block.hip", "host.cpp"]
+SOURCES = ["api.hip", "route.hip", "expert.hip", "expert_bf16.hip", "weights.hip", "block.hip", "host.cpp"]
 ARCH = os.environ.get("KMOE_OFFLOAD_ARCH", "gfx950")
 
 

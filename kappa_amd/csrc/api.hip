@@ -40,6 +40,9 @@ kmoe_status expert_stage(const kmoe_desc& d, int stages, const void* x, const in
   if (packed_ok(d, packed)) {
     e = launch_expert_packed(d, chain_of(d), family_of(d), stages, x, offsets, active, sorted_token, *packed,
                              h_sorted, y_sorted, st, h_scale);
+  } else if (expert_w16_fits(d, stages, x, gate, up, down, h_sorted, y_sorted)) {
+    e = launch_expert_w16(d, chain_of(d), family_of(d), stages, x, offsets, active, sorted_token, gate, up, down,
+                          h_sorted, y_sorted, st);
   } else {
     e = launch_expert_generic(d, chain_of(d), stages, x, sorted_token, sorted_expert, gate, up, down, h_sorted,
                               y_sorted, st);

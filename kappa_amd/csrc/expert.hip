@@ -19,6 +19,7 @@
 #include <atomic>
 
 #include "common.h"
+#include "expert_dev.h"
 #include "launch.h"
 #include "route_dev.h"
 
@@ -27,13 +28,6 @@ namespace kmoe {
 // ---------------------------------------------------------------------------
 // helpers
 // ---------------------------------------------------------------------------
-// two floats -> one dword of bf16 (RNE), a in the low half: one v_cvt_pk_bf16_f32
-__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
-}
-
 // 16 int8 -> bf16(q * s) (s already rounded to bf16), one packed pair at a time.
 // Each byte is biased to u = q + 128 (one XOR per four bytes) and converted by
 // v_cvt_f32_ubyteN; fma(u, s, -128 s) is then q * s exactly (both terms are
@@ -85,83 +79,6 @@ __device__ __forceinline__ void weights16(const uint4 q, const float s, bf16x8& 
 template <int CH>
 __device__ __forceinline__ float chain_scale(float s) {
   return CH == kChainAct ? round_bf16(s) : s;
-}
-
-__device__ __forceinline__ bf16x8 as_bf16x8(const uint4 v) { return __builtin_bit_cast(bf16x8, v); }
-
-// 16 bytes with a nontemporal load: for data a kernel reads exactly once, such
-// as the decode weights (streaming reads this way sustain ~7.1 TB/s on MI355X
-// against ~6.3 TB/s for ordinary loads, which also allocate in the caches)
-__device__ __forceinline__ uint4 load_stream16(const int8_t* p) {
-  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-  return uint4{v.x, v.y, v.z, v.w};
-}
-
-__device__ __forceinline__ floatx4 mfma16(const bf16x8 a, const bf16x8 b, const floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// Block-wide tile prefix over experts: mtp[e] = sum_{e' < e} ceil(min(group_size[e'], cap) / BM), mtp[E] = total.
-// The first 256 threads compute it (E <= 1024); blockDim.x must be a multiple of 64, at least 256.
-// wsum: 4 ints of LDS scratch. offs (optional, E + 1 ints of LDS): a copy of offsets, so
-// the caller's later lookups of its expert's row range are LDS reads, not another global
-// round trip.
-template <int BM>
-__device__ void tile_prefix(const int32_t* __restrict__ offsets, int E, int cap, int* mtp, int* wsum,
-                            int* offs = nullptr) {
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  int c[4];
-  int local = 0, incl = 0;
-  if (tid < 256) {
-    // offsets[4 tid .. 4 tid + 4], clamped to the array: five loads in flight
-    // together (guarded loads would each wait a round trip of their own)
-    int o[5];
-#pragma unroll
-    for (int i = 0; i < 5; ++i) o[i] = offsets[min(tid * 4 + i, E)];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = tid * 4 + i;
-      c[i] = e < E ? (min(o[i + 1] - o[i], cap) + BM - 1) / BM : 0;
-      if (offs != nullptr && e <= E) offs[e] = o[i];
-      local += c[i];
-    }
-    if (offs != nullptr && tid * 4 + 4 == E) offs[E] = o[4];
-    incl = local;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int v = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += v;
-    }
-    if (lane == 63) wsum[wv] = incl;
-  }
-  __syncthreads();
-  if (tid < 256) {
-    int base = 0;
-    for (int w = 0; w < wv; ++w) base += wsum[w];
-    int run = base + incl - local;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = tid * 4 + i;
-      if (e < E) mtp[e] = run;
-      run += c[i];
-    }
-    if (tid == 255) mtp[E] = base + incl;
-  }
-  __syncthreads();
-}
-
-// largest e in [0, E) with mtp[e] <= v (mtp non-decreasing, mtp[0] = 0)
-__device__ __forceinline__ int tile_expert(const int* mtp, int E, int v) {
-  int lo = 0, hi = E - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (mtp[mid] <= v)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
 }
 
 // ---------------------------------------------------------------------------
@@ -836,50 +753,6 @@ __global__ __launch_bounds__(256, 2) void k_prefill(int D, int I, int E, const u
 // go to the same XCD, so the row tiles of one expert share
 // its weights, and the column tiles its rows, in that XCD's L2.
 // ---------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void lds_void;
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const lds_void*)p; }
-
-// 16 bytes per lane from global memory (sbase + voff) into LDS at lds + 16 * lane.
-// sbase and lds must be wave-uniform. The LDS address goes through M0: the
-// asm keeps the caller's M0 (saved and restored, so no clobber of a register
-// the compiler reserves) and puts one wait state between the SALU write of M0
-// and the LDS-DMA load that reads it (a gfx9 hazard the compiler does not see
-// inside inline asm).
-__device__ __forceinline__ void dma16(uint32_t voff, const void* sbase, uint32_t lds) {
-  uint32_t m0save;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-      : "=&s"(m0save)
-      : "v"(voff), "s"(sbase), "s"(lds)
-      : "memory");
-}
-// The same with the nontemporal hint, for weights no other tile re-reads.
-__device__ __forceinline__ void dma16_stream(uint32_t voff, const void* sbase, uint32_t lds) {
-  uint32_t m0save;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
-      : "=&s"(m0save)
-      : "v"(voff), "s"(sbase), "s"(lds)
-      : "memory");
-}
-
-// Wait until at most N of this wave's vector-memory loads are outstanding and
-// its LDS reads are done, then a workgroup barrier. The "memory" clobber keeps
-// every LDS access on its side.
-template <int N>
-__device__ __forceinline__ void vm_barrier() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// Element offset of 16-byte piece p of row r in an A stage: [row][8 x 16 B],
-// pieces XOR-swizzled by (r >> 1) & 7. A row is half the 256-byte bank width,
-// so this puts the 16 rows one fragment read touches on 16 distinct 16-byte
-// bank groups.
-__device__ __forceinline__ int a_piece(int r, int p) { return p ^ (r & 7); }
-__device__ __forceinline__ int a_swz(int r, int p) { return r * 64 + (a_piece(r, p) << 3); }
-
 constexpr int kGemmRows = 128;                // rows per tile (the 128-row form)
 constexpr int kGemmB = 16 * 1024;             // B stage: 16 cells x 64 k x 16 columns int8
 constexpr int kGemmBJ = 4;                    // B loads per wave per chunk (one cell each)

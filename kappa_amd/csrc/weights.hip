@@ -37,11 +37,15 @@ __device__ __forceinline__ void transpose4x4(const uint32_t* r, uint32_t* c) {
 __global__ __launch_bounds__(256) void k_pack(int Kd, int N, int W, const int8_t* __restrict__ src0,
                                               const int8_t* __restrict__ src1, int8_t* __restrict__ dst) {
   typedef uint32_t __attribute__((aligned(1))) u32_any;
-  const int quad = blockIdx.x * 64 + (threadIdx.x & 63);  // four columns
   const int KG = Kd >> 4;
-  const int kg = blockIdx.y * 4 + (threadIdx.x >> 6);
-  const int which = W == 2 ? (int)(blockIdx.z & 1) : 0;
-  const int64_t e = W == 2 ? blockIdx.z >> 1 : blockIdx.z;
+  // blocks over columns (fastest), k groups, matrices (one-dimensional: either extent
+  // may exceed a grid's other dimensions)
+  const uint32_t nx = ((N >> 2) + 63) >> 6, ny = (KG + 3) >> 2;
+  const uint32_t bx = blockIdx.x % nx, bz = blockIdx.x / nx / ny, by = blockIdx.x / nx - bz * ny;
+  const int quad = bx * 64 + (threadIdx.x & 63);  // four columns
+  const int kg = by * 4 + (threadIdx.x >> 6);
+  const int which = W == 2 ? (int)(bz & 1) : 0;
+  const int64_t e = W == 2 ? bz >> 1 : bz;
   if (quad * 4 >= N || kg >= KG) return;
   const int8_t* src = (which ? src1 : src0) + (e * Kd + (int64_t)kg * 16) * N + quad * 4;
   uint32_t r[16];
@@ -133,8 +137,10 @@ __device__ __forceinline__ float channel_scale(float amax) {
 // and store phases follow each other; persistent blocks that request the next
 // item's sweeps while storing measured 179 us per matrix against 167.
 template <typename Wt, int SW>
-__global__ __launch_bounds__(1024, SW == 8 ? 8 : 4) void k_quantize_strip(int E, int Kd, int N, const Wt* __restrict__ w,
-                                                         int8_t* __restrict__ q, float* __restrict__ s) {
+__global__ __launch_bounds__(1024, SW == 8 ? 8 : 4) void k_quantize_strip(int E, int Kd, int N,
+                                                                          const Wt* __restrict__ w,
+                                                                          int8_t* __restrict__ q,
+                                                                          float* __restrict__ s) {
   constexpr int VPT = 16 / sizeof(Wt);  // columns per thread
   constexpr int TPR = 64 / VPT;         // threads per row
   constexpr int RPS = 1024 / TPR;       // rows per sweep
@@ -286,7 +292,8 @@ hipError_t launch_prepack(const kmoe_desc& d, const kmoe_weight& gate, const kmo
                           const kmoe_packed_experts& p, hipStream_t st) {
   const int E = (int)d.num_experts, D = (int)d.hidden, I = (int)d.intermediate;
   auto pack = [&](int Kd, int N, int W, const kmoe_weight& w0, const kmoe_weight& w1, void* dst) {
-    hipLaunchKernelGGL(k_pack, dim3((N / 4 + 63) / 64, (Kd / 16 + 3) / 4, E * W), dim3(256), 0, st, Kd, N, W,
+    hipLaunchKernelGGL(k_pack, dim3((unsigned)((int64_t)((N / 4 + 63) / 64) * ((Kd / 16 + 3) / 4) * E * W)), dim3(256), 0,
+                       st, Kd, N, W,
                        reinterpret_cast<const int8_t*>(w0.values), reinterpret_cast<const int8_t*>(w1.values),
                        reinterpret_cast<int8_t*>(dst));
     return hipGetLastError();
@@ -325,7 +332,7 @@ template <typename W>
 static bool quantize_strip_fits(int64_t E, int64_t Kd, int64_t N, const void* w, const void* q) {
   const int64_t vpt = 16 / sizeof(W);
   return N % vpt == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % vpt == 0 &&
-         E * ((N + 127) / 128) < ((int64_t)1 << 26) && Kd < ((int64_t)1 << 31) / (int64_t)sizeof(W) / N;
+         E * ((N + 127) / 128) < ((int64_t)1 << 20) && Kd < ((int64_t)1 << 31) / (int64_t)sizeof(W) / N;
 }
 
 template <typename W>

@@ -734,7 +734,7 @@ __global__ __launch_bounds__(256, 2) void k_prefill(int D, int I, int E, const u
 //
 // Both operands reach LDS by direct global->LDS loads (global_load_lds_dwordx4):
 // A (activation rows, gathered by token for gate/up) in a 2-stage ring as
-// [row][8 x 16 B] with the 16-byte pieces XOR-swizzled by row, B (the packed
+// [row][8 x 16 B] with the 16-byte pieces swizzled by row (a_at), B (the packed
 // cells, whose 16 bytes per lane are exactly one lane's MFMA fragment of one
 // column) in a 3-stage ring, so the weights, which come from HBM, are
 // requested two chunks ahead and the activation rows, mostly L2 hits, one
@@ -747,8 +747,9 @@ __global__ __launch_bounds__(256, 2) void k_prefill(int D, int I, int E, const u
 // itself (vmcnt is in-order), then a barrier publishes the stage and frees
 // the ones read last.
 //
-// Rows past the expert's end are loaded from a clamped copy of row 0 and never
-// stored; the loop body is instantiated for 1 to 8 (10) active 16-row tiles.
+// Rows past the expert's end are loaded from a clamped copy of row 0 (up to the
+// next multiple of 16) and never stored; the loop body is instantiated for 1 to 8
+// (10) active 16-row tiles.
 // Work items are ordered (expert, column tile, row tile) and consecutive items
 // go to the same XCD, so the row tiles of one expert share
 // its weights, and the column tiles its rows, in that XCD's L2.
@@ -807,11 +808,14 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmLoads<GemmSha
 #pragma unroll
     for (int g = 0; g < 4; ++g) acc[mi][g] = floatx4{0.f, 0.f, 0.f, 0.f};
 
+  // rows past the tile's last 16-row block are not loaded
+  auto a_on = [&](int j) { return 32 * j + 8 * wv < 16 * MT; };
   auto issue_a = [&](int c) {
-    const uint32_t st = lds0 + (uint32_t)((c & 1) * kGemmA + wv * kGemmAJ * 1024);
+    const uint32_t st = lds0 + (uint32_t)((c & 1) * kGemmA + wv * 1024);
     const uint16_t* abase = src + (PL == 2 ? (c & 1) * (KCW * 64) + (c >> 1) * 64 : c * 64);
 #pragma unroll
-    for (int j = 0; j < kGemmAJ; ++j) dma16(gl.avoff[j], abase, st + j * 1024);
+    for (int j = 0; j < kGemmAJ; ++j)
+      if (a_on(j)) dma16(gl.avoff[j], abase, st + j * 4096);
   };
   auto issue_b = [&](int b) {
     const uint32_t st = lds0 + (uint32_t)(kGemmNA * kGemmA + (b % kGemmNB) * kGemmB + wv * 4096);
@@ -843,9 +847,37 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmLoads<GemmSha
     vm_barrier<0>();
   }
   bf16x8 lo[4], hi[4];
+  // A chunk's 2 MT activation fragments, in the order (st, mi), three in flight: the
+  // first three are read with the raw weights, before the conversion, and the
+  // MFMAs of one cover the read of the third after it. The MFMAs run at raised
+  // wave priority, so of the two blocks of a CU one multiplies while the other
+  // converts instead of both doing the same. Same sums, layers before -> after (two
+  // interleaved rounds, with the fragment order of a_at): 30B-A3B T = 2048 / 4096
+  // 288 -> 281 and 457 -> 447 us, 235B-A22B T = 2048 808 -> 780 us. The priority
+  // alone, or the prefetch without the fixed order, gained nothing; the static
+  // priority of one block over the other lost 2%. The 64-row form (three blocks per
+  // CU, bound by the weight stream) is left to the compiler's order: held to this
+  // one, 30B-A3B T = 333 took 165 us instead of 163.
+  constexpr bool kOrdered = RW > 64;
+  constexpr int NK = 2 * MT;
+  constexpr int PF = kOrdered ? (NK < 3 ? NK : 3) : 1;
   for (int c = 0; c < KC; ++c) {
     const int b = PL == 2 ? c >> 1 : c;
+    const bool fresh = PL == 1 || (c & 1) == 0;  // a new weight chunk
     bool b_ahead = false;  // a weight chunk issued this iteration
+    uint4 raw[4];
+    if (fresh) {
+      const uint8_t* bp = bring + (b % kGemmNB) * kGemmB + wv * 4096 + lane * 16;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) raw[g] = *reinterpret_cast<const uint4*>(bp + g * 1024);
+    }
+    const uint16_t* As = reinterpret_cast<const uint16_t*>(smem + (c & 1) * kGemmA);
+    auto a_read = [&](int k) {
+      return *reinterpret_cast<const bf16x8*>(As + a_at<1>((k % MT) * 16 + (lane & 15), 2 * (lane >> 4) + k / MT));
+    };
+    bf16x8 af[PF];
+#pragma unroll
+    for (int k = 0; k < PF; ++k) af[k] = a_read(k);
     if (c + 1 < KC) issue_a(c + 1);
     if (PL == 1 && c + kAhead < KC) {
       issue_b(c + kAhead);
@@ -855,25 +887,27 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmLoads<GemmSha
       issue_b(b + 1);
       b_ahead = true;
     }
-    if (PL == 1 || (c & 1) == 0) {
-      uint4 raw[4];
-      const uint8_t* bp = bring + (b % kGemmNB) * kGemmB + wv * 4096 + lane * 16;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) raw[g] = *reinterpret_cast<const uint4*>(bp + g * 1024);
+    if (fresh) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) weights16<CH>(raw[g], gl.sc[g], lo[g], hi[g]);
     }
-    const uint16_t* As = reinterpret_cast<const uint16_t*>(smem + (c & 1) * kGemmA);
+    if constexpr (kOrdered) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      const int p = 2 * (lane >> 4) + st;
+    for (int k = 0; k < NK; ++k) {
+      // weights as the first operand: the accumulator tile is the output
+      // transposed, so a lane holds four consecutive columns of one row
 #pragma unroll
-      for (int mi = 0; mi < MT; ++mi) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(As + a_swz(mi * 16 + (lane & 15), p));
-        // weights as the first operand: the accumulator tile is the output
-        // transposed, so a lane holds four consecutive columns of one row
+      for (int g = 0; g < 4; ++g) acc[k % MT][g] = mfma16(k < MT ? lo[g] : hi[g], af[k % PF], acc[k % MT][g]);
+      if (k + PF < NK) af[k % PF] = a_read(k + PF);
+    }
+    if constexpr (kOrdered) __builtin_amdgcn_s_setprio(0);
+    // the order the compiler is held to (it otherwise reads a fragment right before its
+    // MFMAs and waits for it): four MFMAs, the next read, ...
+    if constexpr (kOrdered && PL == 1) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) acc[mi][g] = mfma16(st ? hi[g] : lo[g], a, acc[mi][g]);
+      for (int k = 0; k < NK; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
+        if (k + PF < NK) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
     }
     if (c + 1 < KC) {
@@ -965,10 +999,11 @@ __device__ __forceinline__ void gemm_tile_i8(uint8_t* smem, const GemmLoads<Gemm
     }
   // chunk c's A and weights both in stage c % depth
   auto issue = [&](int c) {
-    const uint32_t sa = lds0 + (uint32_t)((c % kGemmNA) * kGemmA + wv * kGemmAJ * 1024);
+    const uint32_t sa = lds0 + (uint32_t)((c % kGemmNA) * kGemmA + wv * 1024);
     const uint16_t* abase = src + c * 64;
 #pragma unroll
-    for (int j = 0; j < kGemmAJ; ++j) dma16(gl.avoff[j], abase, sa + j * 1024);
+    for (int j = 0; j < kGemmAJ; ++j)
+      if (32 * j + 8 * wv < 16 * MT) dma16(gl.avoff[j], abase, sa + j * 4096);
     const uint32_t sb = lds0 + (uint32_t)(kGemmNA * kGemmA + (c % kGemmNB) * kGemmB + wv * 4096);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
@@ -983,8 +1018,9 @@ __device__ __forceinline__ void gemm_tile_i8(uint8_t* smem, const GemmLoads<Gemm
   // and at its end waits for chunk c + 1: the only loads left outstanding are
   // those of the chunks issued after it, kGemmAJ + 4 each.
   constexpr int kAhead = kGemmNA - 1;
-  constexpr int kPer = kGemmAJ + kGemmBJ;
-  static_assert(RW <= 64, "one row scale per lane");
+  // (the fewest a wave issues: the A loads past the tile's rows are skipped)
+  constexpr int kPer = (16 * MT > 56 ? 2 : (16 * MT > 24 ? 1 : 0)) + kGemmBJ;
+  static_assert(RW == 64, "one row scale per lane; two A loads per wave at most");
   // the rows' scales, requested before the chunks (lane r holds row r's; the
   // epilogue shuffles them out), so the epilogue does not wait a round trip
   const float hsv = lane < rows ? hs[row0 + lane] : 0.0f;
@@ -1009,8 +1045,8 @@ __device__ __forceinline__ void gemm_tile_i8(uint8_t* smem, const GemmLoads<Gemm
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi) {
       const int r = mi * 16 + (lane & 15);
-      const int32x4 p1 = *reinterpret_cast<const int32x4*>(As + a_swz(r, lane >> 4));
-      const int32x4 p2 = *reinterpret_cast<const int32x4*>(As + a_swz(r, 4 + (lane >> 4)));
+      const int32x4 p1 = *reinterpret_cast<const int32x4*>(As + a_at<0>(r, lane >> 4));
+      const int32x4 p2 = *reinterpret_cast<const int32x4*>(As + a_at<0>(r, 4 + (lane >> 4)));
       // weights as the first operand: the accumulator tile is the output
       // transposed, so a lane holds four consecutive columns of one row
 #pragma unroll
@@ -1108,12 +1144,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm(int D, int I, int E, const uint
   const int KCW = (GATEUP ? D : I) >> 6;
   const int Ndim = GATEUP ? I : D;
   GemmLoads<Sh::kAJ> gl;
-  // A load j of wave wv covers tile rows 8q .. 8q+7, q = wv * AJ + j: lane -> (row, LDS piece lane % 8)
+  // A load j of wave wv covers tile rows 32 j + 8 wv .. + 7: lane -> (row, LDS slot lane % 8)
 #pragma unroll
   for (int j = 0; j < Sh::kAJ; ++j) {
-    const int r = 8 * (wv * Sh::kAJ + j) + (lane >> 3);
+    const int r = 32 * j + 8 * wv + (lane >> 3);
     const int t = tok[r] >= 0 ? tok[r] : tok[0];
-    gl.avoff[j] = ((uint32_t)t * (uint32_t)Kdim + (uint32_t)(a_piece(r, lane & 7) << 3)) * 2u;
+    gl.avoff[j] = ((uint32_t)t * (uint32_t)Kdim + (uint32_t)(a_piece_at<I8 ? 0 : 1>(r, lane & 7) << 3)) * 2u;
   }
   // this wave's cells: gate/up -> (which = g >> 1, h group nt*8 + 2*wv + (g & 1)); down -> column group nt*16 + 4*wv + g
 #pragma unroll

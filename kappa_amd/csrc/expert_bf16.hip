@@ -29,16 +29,6 @@ namespace {
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-// rows a (even k) and b (odd k) of two columns -> one dword of one column each
-__device__ __forceinline__ uint32_t pair_lo(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
-__device__ __forceinline__ uint32_t pair_hi(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
-
-// eight rows of two columns (one dword per row) -> the operands of the two columns
-__device__ __forceinline__ void transpose2(const uint32_t* r, bf16x8& c0, bf16x8& c1) {
-  c0 = as_bf16x8(uint4{pair_lo(r[0], r[1]), pair_lo(r[2], r[3]), pair_lo(r[4], r[5]), pair_lo(r[6], r[7])});
-  c1 = as_bf16x8(uint4{pair_hi(r[0], r[1]), pair_hi(r[2], r[3]), pair_hi(r[4], r[5]), pair_hi(r[6], r[7])});
-}
-
 // eight rows of four columns (8 bytes per row) -> the operands of the four columns
 __device__ __forceinline__ void transpose4(const u32x2* r, bf16x8* c) {
   uint32_t lo[8], hi[8];
@@ -332,7 +322,7 @@ __device__ __forceinline__ void w16_tile(uint8_t* smem, const W16Loads& gl, int 
       const int p = 2 * (lane >> 4) + st;
 #pragma unroll
       for (int mi = 0; mi < MT; ++mi) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(As + a_swz(mi * 16 + (lane & 15), p));
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(As + a_at<1>(mi * 16 + (lane & 15), p));
 #pragma unroll
         for (int g = 0; g < 4; ++g) acc[mi][g] = mfma16(f[st][g], a, acc[mi][g]);
       }
@@ -436,7 +426,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_w16(int D, int I, int E, const 
   for (int j = 0; j < 2; ++j) {
     const int r = 8 * (wv * 2 + j) + (lane >> 3);
     const int t = tok[r] >= 0 ? tok[r] : tok[0];
-    gl.avoff[j] = ((uint32_t)t * (uint32_t)adim + (uint32_t)(a_piece(r, lane & 7) << 3)) * 2u;
+    gl.avoff[j] = ((uint32_t)t * (uint32_t)adim + (uint32_t)(a_piece_at<1>(r, lane & 7) << 3)) * 2u;
   }
   const int width = GATEUP ? 32 : 64;
   const int col_w = nt * (4 * width) + wv * width;

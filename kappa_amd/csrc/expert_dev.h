@@ -17,6 +17,16 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
 
 __device__ __forceinline__ bf16x8 as_bf16x8(const uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 
+// rows a (even k) and b (odd k) of two columns -> one dword of one column each
+__device__ __forceinline__ uint32_t pair_lo(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+__device__ __forceinline__ uint32_t pair_hi(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
+// eight rows of two columns (one dword per row) -> the operands of the two columns
+__device__ __forceinline__ void transpose2(const uint32_t* r, bf16x8& c0, bf16x8& c1) {
+  c0 = as_bf16x8(uint4{pair_lo(r[0], r[1]), pair_lo(r[2], r[3]), pair_lo(r[4], r[5]), pair_lo(r[6], r[7])});
+  c1 = as_bf16x8(uint4{pair_hi(r[0], r[1]), pair_hi(r[2], r[3]), pair_hi(r[4], r[5]), pair_hi(r[6], r[7])});
+}
+
 // 16 bytes with a nontemporal load: for data a kernel reads exactly once, such
 // as the decode weights (streaming reads this way sustain ~7.1 TB/s on MI355X
 // against ~6.3 TB/s for ordinary loads, which also allocate in the caches)
@@ -129,11 +139,23 @@ __device__ __forceinline__ void vm_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// Element offset of 16-byte piece p of row r in an A stage: [row][8 x 16 B],
-// pieces XOR-swizzled by (r >> 1) & 7. A row is half the 256-byte bank width,
-// so this puts the 16 rows one fragment read touches on 16 distinct 16-byte
-// bank groups.
-__device__ __forceinline__ int a_piece(int r, int p) { return p ^ (r & 7); }
-__device__ __forceinline__ int a_swz(int r, int p) { return r * 64 + (a_piece(r, p) << 3); }
+// An A stage is [row][8 x 16 B]: slot x of row r holds piece x ^ (r & 7) of the row's
+// chunk (int8 planes, kOrder = 0) or, for bf16 chunks (kOrder = 1), piece
+// order(x ^ (r & 7)) with order(y) = 2 (y & 3) + (y >> 2). A fragment read takes
+// the four pieces q, q + 4, .. of the lane groups q: 0..3 or 4..7 of an int8
+// chunk, but every second piece (2 q + st) of a bf16 one, whose order makes them
+// four adjacent slots too. With the even slots as they came the reads counted 3
+// bank-conflict cycles each.
+template <int kOrder>
+__device__ __forceinline__ int a_piece_at(int r, int slot) {
+  const int y = slot ^ (r & 7);
+  return kOrder ? ((y & 3) << 1) | (y >> 2) : y;
+}
+// element offset of piece p of row r
+template <int kOrder>
+__device__ __forceinline__ int a_at(int r, int p) {
+  const int y = kOrder ? (p >> 1) | ((p & 1) << 2) : p;
+  return r * 64 + ((y ^ (r & 7)) << 3);
+}
 
 }  // namespace kmoe

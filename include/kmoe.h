@@ -221,16 +221,16 @@ kmoe_status kmoe_rms_norm(const kmoe_desc* desc, const void* x, const void* scal
  * rounded to x.dtype, block_hist [ceil(T/64), E] int32 (per 64-token chunk
  * expert counts consumed by kmoe_dispatch). `scratch` (optional, may be NULL)
  * of kmoe_route_scratch_bytes(desc) bytes lets a call without logits take the
- * two-phase form when x and the router are bf16, D is 512, 1024, 2048 or
- * 4096, E % 16 == 0 and E <= 256: every logit on the matrix cores, then the
+ * two-phase form when x and the router are bf16, D is a multiple of 256 from 512
+ * to 4096, E % 16 == 0 and E <= 256: every logit on the matrix cores, then the
  * canonical order only for the experts within a rigorous f32 error bound of the
- * K-th (the form kmoe_forward uses from 2048 tokens). Selections, weights and
+ * K-th (the form kmoe_forward uses above 240 tokens). Selections, weights and
  * block_hist are the same either way. */
 kmoe_status kmoe_route(const kmoe_desc* desc, const void* x, const kmoe_weight* router, float* logits,
                        void* scratch, size_t scratch_bytes, int32_t* topk_idx, float* topk_w, int32_t* block_hist,
                        void* stream);
 /* Bytes of scratch the two-phase form of kmoe_route needs (the router
- * transposed to bf16 and its column norms' partial sums). */
+ * transposed to bf16, its column norms' partial sums and the partial logits). */
 kmoe_status kmoe_route_scratch_bytes(const kmoe_desc* desc, size_t* bytes);
 
 /* Stable sort of assignments by expert (kappa/qwen3/ffn_moe.py:189-200, 212):

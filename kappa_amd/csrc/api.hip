@@ -239,8 +239,9 @@ kmoe_status forward_general(const kmoe_desc* desc, const void* x, const void* xi
       KMOE_HIP(launch_rms_norm(*desc, x, norm->scale, norm->scale_bf16 ? KMOE_DTYPE_BF16 : KMOE_DTYPE_F32,
                                           norm->eps, norm->h2, st),
                "rms_norm kernel");
-    if (route_mfma_preferred(*desc, *router))
-      KMOE_HIP(launch_route_mfma(*desc, xin, *router, base + w.route_part, tidx, tw, hist, st), "route kernels");
+    const int64_t scratch = route_mfma_place(*desc, *router, w);
+    if (scratch >= 0)
+      KMOE_HIP(launch_route_mfma(*desc, xin, *router, base + scratch, tidx, tw, hist, st), "route kernels");
     else
       KMOE_HIP(launch_route(*desc, xin, *router, nullptr, tidx, tw, hist, st), "route kernels");
     KMOE_HIP(launch_dispatch(*desc, tidx, hist, gs, off, act, stok, sexp, inv, st), "dispatch kernel");

@@ -61,23 +61,37 @@ size_t route_split_part_floats(const kmoe_desc& d) {
 
 bool route_mfma_fits(const kmoe_desc& d, const kmoe_weight& router) {
   const int64_t D = d.hidden;
-  return enum_value(d.act_dtype) == KMOE_DTYPE_BF16 && enum_value(router.dtype) == KMOE_DTYPE_BF16 &&
-         (D == 512 || D == 1024 || D == 2048 || D == 4096) && d.num_experts % 16 == 0 && d.num_experts <= 256;
+  return enum_value(d.act_dtype) == KMOE_DTYPE_BF16 && enum_value(router.dtype) == KMOE_DTYPE_BF16 && D % 256 == 0 &&
+         D >= 512 && D <= 4096 && d.num_experts % 16 == 0 && d.num_experts <= 256;
 }
 
 bool route_mfma_preferred(const kmoe_desc& d, const kmoe_weight& router) {
-  // (layout() reserves its scratch from 2048 tokens)
-  return route_mfma_fits(d, router) && d.tokens >= 2048;
+  return route_mfma_fits(d, router) && d.tokens >= kRouteOwnScratchTokens;
+}
+
+int64_t route_mfma_place(const kmoe_desc& d, const kmoe_weight& router, const Workspace& w) {
+  if (!route_mfma_fits(d, router)) return -1;
+  if (route_mfma_preferred(d, router)) return (int64_t)w.route_part;
+  return w.route_part - w.h_sorted >= route_mfma_scratch_bytes(d) ? (int64_t)w.h_sorted : -1;
+}
+
+int route_mfma_splits(const kmoe_desc& d) {
+  // blocks of 64 tokens; splits while they still fit the chip's CUs once
+  const int64_t tiles = (d.tokens + 63) / 64;
+  int ks = kmoe::kRouteMaxSplits;
+  while (ks > 1 && tiles * ks > 256) ks >>= 1;
+  return ks;
 }
 
 size_t route_mfma_scratch_offsets(const kmoe_desc& d, int part) {
-  const size_t ED = (size_t)d.num_experts * (size_t)d.hidden;
-  const size_t o1 = align_up(2 * ED);
-  const size_t o2 = o1 + 4 * (((size_t)d.hidden + 255) / 256) * (size_t)d.num_experts;
-  return part == 1 ? o1 : (part == 2 ? o2 : 0);
+  const size_t E = (size_t)d.num_experts, D = (size_t)d.hidden, KS = (size_t)route_mfma_splits(d);
+  const size_t o1 = align_up(2 * E * D);
+  const size_t o2 = align_up(o1 + 4 * KS * E);
+  const size_t o3 = o2 + 4 * KS * (size_t)d.tokens * E;
+  return part == 1 ? o1 : (part == 2 ? o2 : (part == 3 ? o3 : 0));
 }
 
-size_t route_mfma_scratch_bytes(const kmoe_desc& d) { return route_mfma_scratch_offsets(d, 2); }
+size_t route_mfma_scratch_bytes(const kmoe_desc& d) { return route_mfma_scratch_offsets(d, 3); }
 
 bool is_float(kmoe_dtype t) {
   const int v = enum_value(t);
@@ -190,10 +204,11 @@ Workspace layout(const kmoe_desc& d, bool block) {
   // the f32 chain keeps h as two bf16 planes per row for bf16 activations
   w.h_sorted = take((chain_of(d) == kmoe::kChainF32 && d.act_dtype == KMOE_DTYPE_BF16 ? 4 : act) * M * I);
   w.y_sorted = take(act * M * D);
-  // the split router's group partials, or above its range the two-phase
-  // router's scratch (a bf16 router; the others need none)
+  // the split router's group partials, or from kRouteOwnScratchTokens the
+  // two-phase router's scratch (a bf16 router; the others need none; between the
+  // two it is in h_sorted and y_sorted, route_mfma_place)
   w.route_part = take(T <= (size_t)kSplitRouterMaxTokens ? 4 * route_split_part_floats(d)
-                                                         : (T >= 2048 ? route_mfma_scratch_bytes(d) : 0));
+                                                         : (T >= (size_t)kRouteOwnScratchTokens ? route_mfma_scratch_bytes(d) : 0));
   w.h_scale = take(down_planes_fits(d) ? 4 * M : 0);
   w.normed = take(block ? act * T * D : 0);  // rms_norm(h) for kmoe_forward_block
   w.total = o;

@@ -25,6 +25,7 @@ constexpr int kDispatchBlock = 64;
 constexpr int kMaxExperts = 1024;
 constexpr int kMaxTopK = 64;
 constexpr int kMaxRouterSlices = 64;  // D <= 4096
+constexpr int kRouteMaxSplits = 8;    // blocks that split a two-phase router's reduction
 // Decode kernels keep up to this many 16-row blocks of one expert in registers.
 constexpr int kDecodeMaxRowBlocks = 4;  // T <= 64 tokens
 constexpr int kRowsPathMaxTokens = 128;  // above the decode sizes, the row-group kernels up to this T
@@ -103,23 +104,21 @@ inline int enum_value(const En& e) {
 int route_split_groups(const kmoe_desc& d);
 size_t route_split_part_floats(const kmoe_desc& d);
 // Two-phase router (MFMA logits, canonical recompute of the candidates): the
-// shapes it takes (bf16 activations and router, D one of 512, 1024, 2048,
-// 4096, E % 16 == 0, E <= 256) and its scratch: the router transposed
-// to bf16 [E][8][D/64][8] (offset 0) and the partial sums of squares of its
-// columns [D/256][E] f32 (offset part 1); part 2 is the total.
+// shapes it takes (bf16 activations and router, D a multiple of 256 from 512 to
+// 4096, E % 16 == 0, E <= 256), the splits of its reduction over blocks (KS), and its
+// scratch: the router transposed to bf16 [E][8][D/64][8] (offset 0), the partial sums
+// of squares of its columns [KS][E] f32 (offset part 1) and the partial logits
+// [KS][T][E] f32 (part 2); part 3 is the total.
 bool route_mfma_fits(const kmoe_desc& d, const kmoe_weight& router);
-// Whether kmoe_forward routes with it: it costs about one block's latency per
-// round of blocks (16 tokens per block up to D = 2048, 8 at D = 4096) where the
-// all-VALU k_route grows with T. Alone, with the router in cache, k_route wins
-// up to ~2300 tokens at D = 2048 and ~4000 at D = 4096; inside the layer, where
-// the expert GEMMs have evicted the router, whole layers with the one-phase and
-// the two-phase router (two interleaved rounds) ran 30B-A3B T = 2048 / 2560 /
-// 3072 / 4096 310 / 386 / 436 / 519 against 311 / 376 / 435 / 505 us, 235B-A22B
-// T = 2048 / 3072 / 4096 874 / 1350 / 1696 against 873 / 1338 / 1668 us: even at
-// 2048 tokens, ahead above, for both widths.
-bool route_mfma_preferred(const kmoe_desc& d, const kmoe_weight& router);
+int route_mfma_splits(const kmoe_desc& d);
 size_t route_mfma_scratch_offsets(const kmoe_desc& d, int part);
 size_t route_mfma_scratch_bytes(const kmoe_desc& d);
+// kmoe_forward routes with it above the split router's sizes. From this many tokens
+// the workspace holds a scratch for it (route_mfma_preferred); below, the scratch is in
+// the h_sorted and y_sorted buffers, which nothing uses before the expert
+// kernels, so that calls of up to 291 tokens stay inside the no-allocation scratch.
+constexpr int kRouteOwnScratchTokens = 2048;
+bool route_mfma_preferred(const kmoe_desc& d, const kmoe_weight& router);
 
 // --- status and message ------------------------------------------------------
 // Records the message of a failing status for kmoe_last_error (per thread).
@@ -156,6 +155,10 @@ struct Workspace {
 // (Workspace::h_scale).
 bool down_planes_fits(const kmoe_desc& d);
 Workspace layout(const kmoe_desc& d, bool block);
+// Workspace offset of the two-phase router's scratch for this call; -1 where the
+// all-VALU router runs instead (the shape does not fit, or h_sorted and y_sorted
+// are smaller than the scratch).
+int64_t route_mfma_place(const kmoe_desc& d, const kmoe_weight& router, const Workspace& w);
 
 // --- argument checks ---------------------------------------------------------
 kmoe_status check_desc(const kmoe_desc* d);

@@ -8,6 +8,7 @@
 #include <cmath>
 
 #include "common.h"
+#include "expert_dev.h"
 #include "launch.h"
 #include "norm.h"
 #include "route_dev.h"
@@ -484,78 +485,173 @@ __global__ __launch_bounds__(256) void k_dispatch_scatter(int T, int E, int K, i
 
 
 // ---------------------------------------------------------------------------
-// Two-phase router: bf16 activations and router, D = 64 S with S a power of
-// two from 8 to 64, E % 16 == 0, E <= 256.
+// Two-phase router: bf16 activations and router, D a multiple of 256, E % 16 == 0,
+// E <= 256.
 //
 // Bit-exact top-k needs the canonical logits (k_route's order) only where the
-// ranking is in doubt. Phase 1 computes every logit on the matrix cores
-// (v_mfma_f32_16x16x32_bf16: exact products, f32 sums in the hardware's order):
-// L~[t,e]. The exact sum, the canonical L and L~ differ by at most
-// c * sum_d |x_d r_de| <= c * ||x_t|| * ||r_e|| (Cauchy-Schwarz), where c covers
-// the MFMA's accumulation (taken as up to 2D roundings of up to 2u each,
-// u = 2^-24), the canonical chains and tree (64 + log2 P roundings), the
-// rounding of the norms and of L~ -/+ delta (the host passes c). So L lies in
-// [lo, hi] = [L~ - delta, L~ + delta], delta = c * ||x_t|| * ||r_e|| + 1e-30.
-// Let tau be the K-th largest lo (the search stops at 16 key bits, which can
+// ranking is in doubt. k_route_logits computes every logit on the matrix cores
+// (v_mfma_f32_16x16x32_bf16: exact products, f32 sums in the hardware's order, the
+// reduction split over blocks): L~[t,e]. The exact sum, the canonical L and L~
+// differ by at most c * sum_d |x_d r_de| <= c * ||x_t|| * ||r_e|| (Cauchy-Schwarz),
+// where c covers the MFMA's accumulation and the sums of the splits (taken as up to
+// 2D roundings of up to 2u each, u = 2^-24), the canonical chains and tree (64 +
+// log2 P roundings), the rounding of the norms and of L~ -/+ delta (the host passes
+// c). So L lies in [lo, hi] = [L~ - delta, L~ + delta], delta = c * ||x_t|| * ||r_e|| +
+// 1e-30. Let tau be the K-th largest lo (the search stops at 16 key bits, which can
 // only lower it). An expert whose hi is below tau has K experts strictly above
 // it and cannot be selected, ties included; the top K are among the
-// candidates {e : hi_e >= tau}. Phase 2 recomputes the candidates' logits in
+// candidates {e : hi_e >= tau}. k_route_select recomputes the candidates' logits in
 // the canonical order, ranks them (value descending, ties to the lower index)
 // and takes the softmax of the first K, as wave_topk does. A token with a
 // non-finite L~ or bound takes every expert as a candidate.
 //
-// The router is transposed once per call into rTq [E][8][S][8] bf16: element
+// k_route_logits also writes the router transposed to rTq [E][8][S][8] bf16: element
 // (e, d = 64 s + 8 i + j) at ((e * 8 + i) * S + s) * 8 + j. Eight consecutive
-// hidden indices of one expert (an MFMA B fragment, or eight steps of a slice
-// chain) are one 16-byte load, and the 8-element pieces i of the S slices of
-// one expert are contiguous, so the slice lanes of a chain read 16 S
-// consecutive bytes per step.
+// hidden indices of one expert (its MFMA operand, and eight steps of a slice
+// chain) are one 16-byte piece, and the pieces i of the S slices of one expert are
+// contiguous, so the slice lanes of a chain read 16 S consecutive bytes per step.
+//
+// Both kernels are chains of L2 round trips, not bandwidth: 30B-A3B T = 333 / 1500 /
+// 4096 9 + 15, 11 + 18 and 14 + 21 us, 235B-A22B T = 2048 16 + 33 us. As one kernel (16
+// tokens per block, every block streaming the whole transposed router that a third
+// kernel had prepared) it took 5 + 36 us at 30B-A3B T = 4096 and 5 + 58 us at 235B-A22B
+// T = 2048, and below 2048 tokens the all-VALU router ran (32 / 35 us at T = 333 / 1500,
+// and 5 us for the histograms).
 // ---------------------------------------------------------------------------
-constexpr int kRouteSliceBytes = 144;  // a 64-element bf16 slice of x in LDS, padded by 16 bytes
 
-// Block (e, p): experts 16e .. 16e+15, hidden rows 256p .. 256p+255 (slices
-// 4p .. 4p+3) of the router: rTq (exact; through LDS, so the stores are the
-// 64-byte runs of four slices of one eighth), the partial sums of squares of
-// the 16 columns npart[p][e], and the histograms zeroed. D % 256 == 0.
-__global__ __launch_bounds__(256) void k_router_prep(int D, int E, const uint16_t* __restrict__ r,
-                                                      uint16_t* __restrict__ rtq, float* __restrict__ npart,
-                                                      int32_t* __restrict__ hist, int nhist) {
-  __shared__ float red[4][16];
-  __shared__ __attribute__((aligned(16))) uint16_t tile[16 * 8 * 4 * 8];  // [e][eighth][slice][8]
-  const int e0 = blockIdx.x * 16, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int nb = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x;
-  for (int i = b * 256 + tid; i < nhist; i += nb * 256) hist[i] = 0;
-  const int d = blockIdx.y * 256 + tid, S = D >> 6;
-  const uint4* row = reinterpret_cast<const uint4*>(r + (int64_t)d * E + e0);
-  const uint4 a = row[0], c = row[1];
-  const uint32_t wd[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
-  const int sl = tid >> 6, i8 = (tid >> 3) & 7, j = tid & 7;
-  float sq[16];
+// Block (tile, ks, h): the partial logits of 64 tokens x 128 experts (128 h ..) over
+// reduction steps [ks, ks + 1) * D / 32 / KS (a step is 32 hidden indices):
+// part[ks][t][e]. The block's four waves take its steps in turn, so no wave loads what
+// another does: lane (c, q) reads experts 8 c .. 8 c + 7 of rows 8 q .. 8 q + 7 (16
+// lanes cover 256 consecutive bytes of a row) and pairs rows in registers
+// (transpose2), and 16 bytes of the rows of the four 16-token tiles; U steps are in
+// flight at once, which is a wave's whole share up to 16 steps per block. The router
+// is the first MFMA operand, so a lane ends with 32 consecutive experts of a token
+// of each tile; the waves' sums meet in LDS, wave w finishing tile w. A step's
+// transposed operands are written to rTq by one of the tiles; tile 0 also sums the
+// squares of its router columns: npart[ks][e]. The blocks zero the histograms
+// together. The same work with 32 experts per wave and all steps in each took
+// 17 / 19 us (30B-A3B T = 4096, 235B-A22B T = 2048), 19 / 21 with the token rows staged
+// in LDS, of which the router's 4-byte loads were 9.
+constexpr int kLogitWaves = 4;
+__global__ __launch_bounds__(64 * kLogitWaves, 1) void k_route_logits(
+    int T, int D, int E, int KS, const uint16_t* __restrict__ x, const uint16_t* __restrict__ r,
+    uint16_t* __restrict__ rtq, float* __restrict__ npart, float* __restrict__ part, int32_t* __restrict__ hist,
+    int nhist) {
+  constexpr int U = 4;
+  __shared__ floatx4 red[kLogitWaves][kLogitWaves - 1][8][64];  // [tile][other wave][4-expert run][lane]
+  __shared__ float nred[kLogitWaves][128];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, q = lane >> 4;
+  const int tile = blockIdx.x, tiles = gridDim.x, ks = blockIdx.y;
+  const int t0 = tile * 64, e0 = blockIdx.z * 128;
+  for (int i = ((blockIdx.z * KS + ks) * tiles + tile) * 256 + threadIdx.x; i < nhist;
+       i += gridDim.z * KS * tiles * 256)
+    hist[i] = 0;
+  const int S = D >> 6, steps = (D >> 5) / KS, st0 = ks * steps;
+  const int e = e0 + 8 * c;
+  const bool on = e < E;
+  const uint16_t* xr[4];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint32_t bits = (i & 1) ? (wd[i >> 1] >> 16) : (wd[i >> 1] & 0xffffu);
-    const float v = __uint_as_float(bits << 16);
-    tile[((i * 8 + i8) * 4 + sl) * 8 + j] = (uint16_t)bits;
-    sq[i] = v * v;
+  for (int mi = 0; mi < 4; ++mi) xr[mi] = x + (int64_t)min(t0 + 16 * mi + c, T - 1) * D + 8 * q;
+  floatx4 acc[8][4];
+  float nn[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    nn[j] = 0.0f;
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi) acc[j][mi] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
+  for (int sb = w; sb < steps; sb += kLogitWaves * U) {
+    uint4 a[U][4], b[U][8];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
+    for (int u = 0; u < U; ++u) {
+      if (sb + kLogitWaves * u < steps) {
+        const int k0 = (st0 + sb + kLogitWaves * u) * 32;
+        const uint16_t* rp = r + (int64_t)(k0 + 8 * q) * E + e;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sq[i] += __shfl_xor(sq[i], off, 64);
+        for (int i = 0; i < 8; ++i)
+          b[u][i] = on ? *reinterpret_cast<const uint4*>(rp + (int64_t)i * E) : uint4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi) a[u][mi] = *reinterpret_cast<const uint4*>(xr[mi] + k0);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int sl = sb + kLogitWaves * u;
+      if (sl < steps) {
+        uint32_t rows[4][8];  // [expert pair][row]
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          rows[0][i] = b[u][i].x;
+          rows[1][i] = b[u][i].y;
+          rows[2][i] = b[u][i].z;
+          rows[3][i] = b[u][i].w;
+        }
+        const int d = (st0 + sl) * 32 + 8 * q;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          bf16x8 f[2];
+          transpose2(rows[p], f[0], f[1]);
+          if (sl % tiles == tile && on) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              *reinterpret_cast<uint4*>(rtq + ((int64_t)((e + 2 * p + j) * 8 + ((d & 63) >> 3)) * S + (d >> 6)) * 8) =
+                  __builtin_bit_cast(uint4, f[j]);
+          }
+          if (tile == 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const float lo = __uint_as_float(rows[p][i] << 16), hi = __uint_as_float(rows[p][i] & 0xffff0000u);
+              nn[2 * p] = __builtin_fmaf(lo, lo, nn[2 * p]);
+              nn[2 * p + 1] = __builtin_fmaf(hi, hi, nn[2 * p + 1]);
+            }
+          }
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int mi = 0; mi < 4; ++mi)
+              acc[2 * p + j][mi] = mfma16(f[j], as_bf16x8(a[u][mi]), acc[2 * p + j][mi]);
+        }
+      }
+    }
   }
-  if (lane == 0) {
+  // lane (c, q), register (j, mi, i): token 16 mi + c, expert e0 + 32 q + 8 i + j. Runs of four
+  // experts: run n holds 32 q + 4 n ..
 #pragma unroll
-    for (int i = 0; i < 16; ++i) red[w][i] = sq[i];
+  for (int mi = 0; mi < 4; ++mi) {
+    if (mi == w) continue;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const int i = n >> 1, j = 4 * (n & 1);
+      red[mi][w < mi ? w : w - 1][n][lane] = floatx4{acc[j][mi][i], acc[j + 1][mi][i], acc[j + 2][mi][i], acc[j + 3][mi][i]};
+    }
+  }
+  if (tile == 0) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      nn[j] += __shfl_xor(nn[j], 16, 64);
+      nn[j] += __shfl_xor(nn[j], 32, 64);
+      if (q == 0) nred[w][8 * c + j] = nn[j];
+    }
   }
   __syncthreads();
-  if (tid < 16) npart[(int64_t)blockIdx.y * E + e0 + tid] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
-  // 512 pieces of 16 bytes: piece q = (expert q / 32, eighth (q / 4) % 8, slice q % 4)
+  if (tile == 0 && threadIdx.x < 128 && e0 + (int)threadIdx.x < E)
+    npart[ks * E + e0 + threadIdx.x] =
+        ((nred[0][threadIdx.x] + nred[1][threadIdx.x]) + nred[2][threadIdx.x]) + nred[3][threadIdx.x];
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int q = tid + 256 * k;
-    const int e = q >> 5, ei = (q >> 2) & 7, s4 = q & 3;
-    *reinterpret_cast<uint4*>(rtq + ((int64_t)((e0 + e) * 8 + ei) * S + 4 * blockIdx.y + s4) * 8) =
-        reinterpret_cast<const uint4*>(tile)[q];
+  for (int mi = 0; mi < 4; ++mi) {
+    if (mi != w) continue;
+    const int t = t0 + 16 * mi + c;
+    float* o = part + ((int64_t)ks * T + t) * E + e0 + 32 * q;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const int i = n >> 1, j = 4 * (n & 1);
+      floatx4 v = floatx4{acc[j][mi][i], acc[j + 1][mi][i], acc[j + 2][mi][i], acc[j + 3][mi][i]};
+#pragma unroll
+      for (int k = 0; k < kLogitWaves - 1; ++k) v += red[mi][k][n][lane];
+      if (t < T && e0 + 32 * q + 4 * n < E) *reinterpret_cast<floatx4*>(o + 4 * n) = v;
+    }
   }
 }
 
@@ -565,164 +661,88 @@ __device__ __forceinline__ uint32_t float_key(float v) {
   return (u >> 31) ? ~u : (u | 0x80000000u);
 }
 
-// Block: TB tokens, one wave each. The token rows are staged in LDS first
-// (slice-padded: slice s of row r at r * XRS + s * 144). Phase 1: the
-// 16-token x 16-expert logit tiles over waves (tile = w % NT, and with more
-// waves than tiles the reduction split KS ways, ks = w / NT), A from LDS, B
-// from rTq in batches of 16 steps; partial sums to LDS, and the waves of tile
-// 0 also sum the squares of their rows for ||x||. Phase 2: wave w finishes
-// token w: P lanes per candidate chain (the zero-padded slice count), 64 / P
-// chains side by side.
-template <int EPL, int P, int TB>
-__global__ __launch_bounds__(64 * TB) void k_route_mfma(int T, int D, int E, int K, const uint16_t* __restrict__ x,
-                                                         const uint16_t* __restrict__ rtq,
-                                                         const float* __restrict__ npart, float cbound,
-                                                         int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
-                                                         int32_t* __restrict__ hist, int out_bf16) {
+constexpr int kSelectWaves = 4;        // tokens per block of k_route_select, one wave each
+constexpr int kRouteSliceBytes = 144;  // a 64-element bf16 slice of x in LDS, padded by 16 bytes
+
+// One wave per token (no block barrier): the bound and the candidates from the
+// partial logits, their canonical logits (P lanes per chain, the slice count rounded
+// up to a power of two; 64 / P chains side by side, two rounds of them in flight),
+// rank, softmax, and the per-64-token expert counts.
+template <int EPL, int P>
+__global__ __launch_bounds__(64 * kSelectWaves, EPL <= 2 ? 4 : 2) void k_route_select(
+    int T, int D, int E, int K, int KS, const uint16_t* __restrict__ x, const uint16_t* __restrict__ rtq,
+    const float* __restrict__ npart, const float* __restrict__ part, float cbound, int32_t* __restrict__ topk_idx,
+    float* __restrict__ topk_w, int32_t* __restrict__ hist, int out_bf16) {
   static_assert(EPL <= 4, "experts per lane");
   constexpr int CP = 64 / P;  // chains side by side in a wave
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds8[];
-  __shared__ TopkLds tk[TB];
-  __shared__ float nxp[16][16];  // [ks][row] partial sums of squares
+  __shared__ TopkLds tk[kSelectWaves];
+  __shared__ __attribute__((aligned(16))) uint8_t xlds[kSelectWaves][P * kRouteSliceBytes];
+  __shared__ int32_t cand_lds[kSelectWaves][64 * EPL];
+  __shared__ float cval_lds[kSelectWaves][64 * EPL];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int t0 = blockIdx.x * TB;
-  const int S = D >> 6;
-  const int XRS = S * kRouteSliceBytes + 16;
-  const int NT = E >> 4;
-  const int KS = TB >= NT ? TB / NT : 1;
-  uint8_t* xs = lds8;
-  float* lgp = reinterpret_cast<float*>(lds8 + TB * XRS);
-  const int lgp_floats = TB * 256 > 16 * E ? TB * 256 : 16 * E;
-  int32_t* cand = reinterpret_cast<int32_t*>(lgp + lgp_floats) + w * E;
-  float* cval = reinterpret_cast<float*>(reinterpret_cast<int32_t*>(lgp + lgp_floats) + TB * E) + w * E;
-  // the router columns' partial sums of squares, [D / 256][E], staged with the token rows
-  const int NPD = (D + 255) >> 8;
-  float* npl = reinterpret_cast<float*>(lds8 + TB * XRS) + lgp_floats + 2 * TB * E;
-
-  // ---- phase 1 assignment: tiles tile0, tile0 + tstep, ... over steps [s0, s1) ----
-  // Step st, k-lane kq takes the 8 hidden indices of piece p = 4 st + kq, with
-  // piece p = slice p % S, eighth p / S (any one-to-one map of the reduction
-  // works when A and B follow it): the four k-lanes of an expert then read 64
-  // consecutive bytes of rTq.
-  const int m = lane & 15, kq = lane >> 4;
-  const int nsteps = D >> 5;
-  const int spk = (nsteps + KS - 1) / KS;
-  const bool split = TB >= NT;
-  // with more waves than tiles, waves past KS * NT (NT not dividing TB) sit out
-  const int tile0 = split ? (w < KS * NT ? w % NT : NT) : w;
-  const int tstep = split ? NT : TB;
-  const int ks = split ? w / NT : 0;
-  const int s0 = ks * spk, s1 = min(nsteps, s0 + spk);
-  static_assert((P & (P - 1)) == 0 && P >= 8, "slices: a power of two");
-  constexpr int LP = P == 8 ? 3 : (P == 16 ? 4 : (P == 32 ? 5 : 6));  // log2 S (S == P)
-  auto bload = [&](int tile, int st) {
-    const int p = 4 * st + kq;
-    return *reinterpret_cast<const uint4*>(rtq + ((int64_t)((16 * tile + m) * 8 + (p >> LP)) * P + (p & (P - 1))) * 8);
-  };
-  // router fragments in batches of kRouteBatch steps per wave
-  constexpr int kRouteBatch = 8;
-  uint4 b[kRouteBatch];
-  const bool pre = tile0 < NT && s1 - s0 >= kRouteBatch;
-
-  // ---- the token rows into LDS (rows past T as zeros), the norm partials,
-  // and the first batch of router fragments requested behind them ----
-  {
-    const int cpr = D >> 3;  // 16-byte pieces per row
-    const int per = (TB * cpr) / (64 * TB);  // per thread (D / 512, exact)
-    constexpr int PMAX = TB >= 16 ? 4 : 8;    // the host runs 16 tokens per block up to D = 2048
-    uint4 v[PMAX];
-#pragma unroll
-    for (int k = 0; k < PMAX; ++k) {
-      if (k < per) {
-        const int i = threadIdx.x + k * 64 * TB;
-        const int r = i / cpr, c = i - r * cpr;
-        v[k] = t0 + r < T ? reinterpret_cast<const uint4*>(x + (int64_t)(t0 + r) * D)[c] : uint4{0u, 0u, 0u, 0u};
-      }
-    }
-    if (pre) {
-#pragma unroll
-      for (int j = 0; j < kRouteBatch; ++j) b[j] = bload(tile0, s0 + j);
-    }
-    for (int i = threadIdx.x; i < NPD * E; i += 64 * TB) npl[i] = npart[i];
-#pragma unroll
-    for (int k = 0; k < PMAX; ++k) {
-      if (k < per) {
-        const int i = threadIdx.x + k * 64 * TB;
-        const int r = i / cpr, c = i - r * cpr;
-        *reinterpret_cast<uint4*>(xs + r * XRS + (c >> 3) * kRouteSliceBytes + (c & 7) * 16) = v[k];
-      }
-    }
-  }
-  __syncthreads();
-
-  // ---- phase 1 ----
-  {
-    const uint8_t* xa = xs + (m % TB) * XRS;
-    for (int tile = tile0; tile < NT; tile += tstep) {
-      const int e = 16 * tile + m;
-      floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-      float ss = 0.0f;
-      auto step = [&](int st, const uint4 bb) {
-        const int p = 4 * st + kq;
-        const uint4 a = *reinterpret_cast<const uint4*>(xa + (p & (P - 1)) * kRouteSliceBytes + (p >> LP) * 16);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bb),
-                                                      acc, 0, 0, 0);
-        if (tile == 0) {
-          const uint32_t av[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float lo = __uint_as_float(av[i] << 16), hi = __uint_as_float(av[i] & 0xffff0000u);
-            ss = __builtin_fmaf(lo, lo, ss);
-            ss = __builtin_fmaf(hi, hi, ss);
-          }
-        }
-      };
-      int st = s0;
-      bool have = tile == tile0 && pre;  // b holds steps s0 .. s0 + kRouteBatch - 1
-      for (; st + kRouteBatch <= s1; st += kRouteBatch) {
-        if (!have) {
-#pragma unroll
-          for (int j = 0; j < kRouteBatch; ++j) b[j] = bload(tile, st + j);
-        }
-        have = false;
-#pragma unroll
-        for (int j = 0; j < kRouteBatch; ++j) step(st + j, b[j]);
-      }
-      for (; st < s1; ++st) step(st, bload(tile, st));
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = 4 * kq + j;
-        if (row < TB) lgp[(ks * 16 + row) * E + e] = acc[j];
-      }
-      if (tile == 0) {
-        // row m's squares over this wave's reduction range: the four k-lanes of the row
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
-        if (kq == 0) nxp[ks][m] = ss;
-      }
-    }
-  }
-  __syncthreads();
-
-  // ---- phase 2: wave w, token t0 + w ----
-  const int t = t0 + w;
+  const int t = blockIdx.x * kSelectWaves + w;
   if (t >= T) return;
+  int32_t* cand = cand_lds[w];
+  float* cval = cval_lds[w];
+  const int S = D >> 6;
   const int s = lane % P, g = lane / P;
+  // everything the bound needs, requested together: the lane's slice of x, the
+  // partial logits and the column norms of its experts
+  // (through LDS: read a slice per lane, a row's 16-byte pieces are 128 bytes apart
+  // and every load of the eight touches every cache line of the row)
+  uint8_t* xl = xlds[w];
+  const int pieces = D >> 3;
+  uint4 xv[8];
+#pragma unroll
+  for (int i = 0; i < P / 8; ++i)
+    if (lane + 64 * i < pieces) xv[i] = reinterpret_cast<const uint4*>(x + (int64_t)t * D)[lane + 64 * i];
+  float pl[EPL][kRouteMaxSplits], pn[EPL][kRouteMaxSplits];
+#pragma unroll
+  for (int i = 0; i < EPL; ++i)
+#pragma unroll
+    for (int k = 0; k < kRouteMaxSplits; ++k) {
+      const bool on = k < KS && lane + 64 * i < E;
+      pl[i][k] = on ? part[((int64_t)k * T + t) * E + lane + 64 * i] : 0.0f;
+      pn[i][k] = on ? npart[k * E + lane + 64 * i] : 0.0f;
+    }
+#pragma unroll
+  for (int i = 0; i < P / 8; ++i) {
+    const int pc = lane + 64 * i;
+    if (pc < pieces) *reinterpret_cast<uint4*>(xl + (pc >> 3) * kRouteSliceBytes + (pc & 7) * 16) = xv[i];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    xv[i] = s < S ? *reinterpret_cast<const uint4*>(xl + s * kRouteSliceBytes + 16 * i) : uint4{0u, 0u, 0u, 0u};
   float ss = 0.0f;
-  for (int k2 = 0; k2 < KS; ++k2) ss += nxp[k2][w];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t wd[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float lo = __uint_as_float(wd[j] << 16), hi = __uint_as_float(wd[j] & 0xffff0000u);
+      ss = __builtin_fmaf(lo, lo, ss);
+      ss = __builtin_fmaf(hi, hi, ss);
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < P; o <<= 1) ss += __shfl_xor(ss, o, 64);
   const float nxv = sqrtf(ss);
   float lo[EPL], hi[EPL];
   bool bad = !(nxv <= 3.0e38f);
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
-    const int e = lane + 64 * i;
     lo[i] = -INFINITY;
     hi[i] = -INFINITY;
-    if (e < E) {
-      float v = lgp[w * E + e];
-      for (int k2 = 1; k2 < KS; ++k2) v += lgp[(k2 * 16 + w) * E + e];
-      float n2 = 0.0f;
-      for (int p = 0; p < NPD; ++p) n2 += npl[p * E + e];
+    if (lane + 64 * i < E) {
+      float v = pl[i][0], n2 = pn[i][0];
+#pragma unroll
+      for (int k = 1; k < kRouteMaxSplits; ++k) {
+        v += pl[i][k];
+        n2 += pn[i][k];
+      }
       const float dl = __builtin_fmaf(cbound * nxv, sqrtf(n2), 1e-30f);
       lo[i] = v - dl;
       hi[i] = v + dl;
@@ -761,41 +781,43 @@ __global__ __launch_bounds__(64 * TB) void k_route_mfma(int T, int D, int E, int
   // canonical logits of the candidates: lane s of a group of P runs slice s of
   // candidates g, g + CP, ... (x[64 s ..] times r[64 s ..][e], one fmaf chain
   // from +0), then the pairwise tree over the P slices
-  float xf[64];
-  if (s < S) {
-    const uint8_t* xrow = xs + w * XRS + s * kRouteSliceBytes;
+  auto piece = [&](int c, int i) {
+    // chains past the candidates do no loads and are not stored
+    return s < S && c < nc ? reinterpret_cast<const uint4*>(rtq + ((int64_t)cand[c] * 8 * S + s) * 8)[(int64_t)i * S]
+                           : uint4{0u, 0u, 0u, 0u};
+  };
+  for (int cb = 0; cb < nc; cb += 2 * CP) {
+    const int c0 = cb + g, c1 = cb + CP + g;
+    uint4 r0[8], r1[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const uint4 v = *reinterpret_cast<const uint4*>(xrow + 16 * q);
-      const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
+    for (int i = 0; i < 8; ++i) {
+      r0[i] = piece(c0, i);
+      r1[i] = piece(c1, i);
+    }
+    float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        xf[8 * q + 2 * i] = __uint_as_float(wd[i] << 16);
-        xf[8 * q + 2 * i + 1] = __uint_as_float(wd[i] & 0xffff0000u);
+    for (int i = 0; i < 8; ++i) {
+      // (x stays packed across the rounds: its 64 floats would cost half the waves)
+      asm volatile("" : "+v"(xv[i].x), "+v"(xv[i].y), "+v"(xv[i].z), "+v"(xv[i].w));
+      const uint32_t xw[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+      const uint32_t w0[4] = {r0[i].x, r0[i].y, r0[i].z, r0[i].w};
+      const uint32_t w1[4] = {r1[i].x, r1[i].y, r1[i].z, r1[i].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float xl = __uint_as_float(xw[j] << 16), xh = __uint_as_float(xw[j] & 0xffff0000u);
+        a0 = __builtin_fmaf(xl, __uint_as_float(w0[j] << 16), a0);
+        a1 = __builtin_fmaf(xl, __uint_as_float(w1[j] << 16), a1);
+        a0 = __builtin_fmaf(xh, __uint_as_float(w0[j] & 0xffff0000u), a0);
+        a1 = __builtin_fmaf(xh, __uint_as_float(w1[j] & 0xffff0000u), a1);
       }
     }
-  }
-  for (int c = g; c < ((nc + CP - 1) / CP) * CP; c += CP) {
-    float acc = 0.0f;
-    if (s < S && c < nc) {
-      // chains past the candidates do no loads and are not stored
-      const uint4* rp = reinterpret_cast<const uint4*>(rtq + ((int64_t)cand[c] * 8 * S + s) * 8);
-      uint4 rv[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) rv[i] = rp[(int64_t)i * S];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t wd[4] = {rv[i].x, rv[i].y, rv[i].z, rv[i].w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc = __builtin_fmaf(xf[8 * i + 2 * j], __uint_as_float(wd[j] << 16), acc);
-          acc = __builtin_fmaf(xf[8 * i + 2 * j + 1], __uint_as_float(wd[j] & 0xffff0000u), acc);
-        }
-      }
+    for (int st = 1; st < P; st <<= 1) {
+      a0 = a0 + __shfl_down(a0, st, P);
+      a1 = a1 + __shfl_down(a1, st, P);
     }
-#pragma unroll
-    for (int st = 1; st < P; st <<= 1) acc = acc + __shfl_down(acc, st, P);
-    if (s == 0 && c < nc) cval[c] = acc;
+    if (s == 0 && c0 < nc) cval[c0] = a0;
+    if (s == 0 && c1 < nc) cval[c1] = a1;
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1110,55 +1132,58 @@ hipError_t launch_dispatch(const kmoe_desc& d, const int32_t* topk_idx, const in
   return hipGetLastError();
 }
 
-// Two-phase router: the prep kernel (router transposed to rTq, column-norm
-// partials, histograms zeroed), then the MFMA logits, the candidates'
-// canonical logits, top-k, softmax and the per-64-token expert counts
-// (launch_dispatch reads them as it reads k_dispatch_count's).
-template <int EPL, int P, int TB>
-static void launch_route_mfma_k(const kmoe_desc& d, const uint16_t* x, const uint16_t* rtq, const float* npart,
-                                float cb, int32_t* topk_idx, float* topk_w, int32_t* hist, hipStream_t st) {
-  const int T = (int)d.tokens, D = (int)d.hidden, E = (int)d.num_experts, K = (int)d.top_k;
-  const int XRS = (D / 64) * kRouteSliceBytes + 16;
-  const int lgp = TB * 256 > 16 * E ? TB * 256 : 16 * E;
-  const size_t lds = (size_t)TB * XRS + 4 * ((size_t)lgp + 2 * (size_t)TB * E + (size_t)((D + 255) / 256) * E);
-  hipLaunchKernelGGL((k_route_mfma<EPL, P, TB>), dim3((T + TB - 1) / TB), dim3(64 * TB), lds, st, T, D, E, K, x, rtq,
-                     npart, cb, topk_idx, topk_w, hist, d.act_dtype == KMOE_DTYPE_BF16 ? 1 : 0);
-}
-
-// P lanes per candidate chain (the slice count rounded up to a power of two);
-// 16 tokens per block up to D = 2048, 8 above (the staged rows fit LDS).
+// Two-phase router: the partial logits (with the transposed router, its column
+// norms and the histograms zeroed), then the bound, the candidates' canonical
+// logits, top-k, softmax and the per-64-token expert counts (launch_dispatch
+// reads them as it reads k_dispatch_count's).
 template <int EPL>
-static void route_mfma_p(const kmoe_desc& d, const uint16_t* x, const uint16_t* rtq, const float* npart, float cb,
-                         int32_t* topk_idx, float* topk_w, int32_t* hist, hipStream_t st) {
-  const int S = (int)(d.hidden / 64);
-  if (S <= 8) return launch_route_mfma_k<EPL, 8, 16>(d, x, rtq, npart, cb, topk_idx, topk_w, hist, st);
-  if (S <= 16) return launch_route_mfma_k<EPL, 16, 16>(d, x, rtq, npart, cb, topk_idx, topk_w, hist, st);
-  if (S <= 32) return launch_route_mfma_k<EPL, 32, 16>(d, x, rtq, npart, cb, topk_idx, topk_w, hist, st);
-  return launch_route_mfma_k<EPL, 64, 8>(d, x, rtq, npart, cb, topk_idx, topk_w, hist, st);
+static void route_select_p(const kmoe_desc& d, int KS, const uint16_t* x, const uint16_t* rtq, const float* npart,
+                           const float* part, float cb, int32_t* topk_idx, float* topk_w, int32_t* hist,
+                           hipStream_t st) {
+  const int T = (int)d.tokens, D = (int)d.hidden, E = (int)d.num_experts, K = (int)d.top_k;
+  const dim3 grid((T + kSelectWaves - 1) / kSelectWaves), block(64 * kSelectWaves);
+  const int out_bf16 = d.act_dtype == KMOE_DTYPE_BF16 ? 1 : 0;
+  const int S = D / 64;
+  // P lanes per candidate chain: the slice count rounded up to a power of two
+  if (S <= 8)
+    hipLaunchKernelGGL((k_route_select<EPL, 8>), grid, block, 0, st, T, D, E, K, KS, x, rtq, npart, part, cb, topk_idx,
+                       topk_w, hist, out_bf16);
+  else if (S <= 16)
+    hipLaunchKernelGGL((k_route_select<EPL, 16>), grid, block, 0, st, T, D, E, K, KS, x, rtq, npart, part, cb, topk_idx,
+                       topk_w, hist, out_bf16);
+  else if (S <= 32)
+    hipLaunchKernelGGL((k_route_select<EPL, 32>), grid, block, 0, st, T, D, E, K, KS, x, rtq, npart, part, cb, topk_idx,
+                       topk_w, hist, out_bf16);
+  else
+    hipLaunchKernelGGL((k_route_select<EPL, 64>), grid, block, 0, st, T, D, E, K, KS, x, rtq, npart, part, cb, topk_idx,
+                       topk_w, hist, out_bf16);
 }
 
 hipError_t launch_route_mfma(const kmoe_desc& d, const void* x, const kmoe_weight& r, void* scratch,
                              int32_t* topk_idx, float* topk_w, int32_t* hist, hipStream_t st) {
   const int T = (int)d.tokens, D = (int)d.hidden, E = (int)d.num_experts;
+  const int KS = route_mfma_splits(d);
   char* base = reinterpret_cast<char*>(scratch);
   uint16_t* rtq = reinterpret_cast<uint16_t*>(base);
   float* npart = reinterpret_cast<float*>(base + route_mfma_scratch_offsets(d, 1));
+  float* part = reinterpret_cast<float*>(base + route_mfma_scratch_offsets(d, 2));
   const int nhist = ((T + kDispatchBlock - 1) / kDispatchBlock) * E;
-  hipLaunchKernelGGL(k_router_prep, dim3(E / 16, (D + 255) / 256), dim3(256), 0, st, D, E,
-                     reinterpret_cast<const uint16_t*>(r.values), rtq, npart, hist, nhist);
+  const uint16_t* xb = reinterpret_cast<const uint16_t*>(x);
+  const uint16_t* rb = reinterpret_cast<const uint16_t*>(r.values);
+  hipLaunchKernelGGL(k_route_logits, dim3((T + 63) / 64, KS, (E + 127) / 128), dim3(64 * kLogitWaves), 0, st, T, D, E,
+                     KS, xb, rb, rtq, npart, part, hist, nhist);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   // the error bound's constant, relative to ||x|| ||r_e||: the MFMA sums as up
   // to 2D roundings of up to 2u, the canonical chains and tree, the norms and
   // lo / hi, with room to spare
   const float cb = (float)std::ldexp(4.0 * D + 512.0, -24);
-  const uint16_t* xb = reinterpret_cast<const uint16_t*>(x);
   if (E <= 64)
-    route_mfma_p<1>(d, xb, rtq, npart, cb, topk_idx, topk_w, hist, st);
+    route_select_p<1>(d, KS, xb, rtq, npart, part, cb, topk_idx, topk_w, hist, st);
   else if (E <= 128)
-    route_mfma_p<2>(d, xb, rtq, npart, cb, topk_idx, topk_w, hist, st);
+    route_select_p<2>(d, KS, xb, rtq, npart, part, cb, topk_idx, topk_w, hist, st);
   else
-    route_mfma_p<4>(d, xb, rtq, npart, cb, topk_idx, topk_w, hist, st);
+    route_select_p<4>(d, KS, xb, rtq, npart, part, cb, topk_idx, topk_w, hist, st);
   return hipGetLastError();
 }
 

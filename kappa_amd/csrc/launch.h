@@ -104,7 +104,6 @@ hipError_t launch_gateup_routed(const kmoe_desc& d, int chain, const float* part
                                 const DispatchOut& dout, hipStream_t st);
 
 // block.hip
-size_t rms_norm_lds_bytes(int64_t D);
 hipError_t launch_rms_norm(const kmoe_desc& d, const void* h, const void* scale, kmoe_dtype scale_dtype, float eps,
                            void* out, hipStream_t st);
 

@@ -6,48 +6,95 @@
 
 namespace kmoe {
 
-constexpr int kNormBatch = 32;  // row elements per lane in flight (a 2048-wide row in one batch)
+// A row of D elements staged in LDS for its reduction: slices of 64 elements, 16 bytes
+// apart more than their size, so that the lanes' slices start in distinct banks
+// and stay 16-byte aligned.
+template <typename A>
+struct NormRow {
+  static constexpr int kPiece = 16 / sizeof(A);             // elements of a 16-byte piece
+  static constexpr int kSlice = kRouterSlice + kPiece;      // elements per staged slice
+  static constexpr int kPieces = 64 * kRouterSlice / kPiece / 64;  // pieces per lane of the widest row (D = 4096)
+  __host__ __device__ static size_t bytes(int D) {
+    return (size_t)((D + kRouterSlice - 1) / kRouterSlice) * kSlice * sizeof(A);
+  }
+  __device__ __forceinline__ static int at(int d) { return (d >> 6) * kSlice + (d & 63); }
+  // rows that move in 16-byte pieces
+  __device__ __forceinline__ static bool pieces(const A* src, int D) {
+    return D % kRouterSlice == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+  }
+  __device__ __forceinline__ static void unpack(const uint4& v, float* f) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (sizeof(A) == 2) {
+        f[2 * i] = __uint_as_float(w[i] << 16);
+        f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+      } else {
+        f[i] = __uint_as_float(w[i]);
+      }
+    }
+  }
+};
 
-// LDS floats one wave needs to stage a row of D elements: [slice][65].
-__host__ __device__ inline int norm_row_floats(int D) { return ((D + kRouterSlice - 1) / kRouterSlice) * (kRouterSlice + 1); }
-
-// One wave: stage the row src[0..D) in LDS as f32 row[slice][65] (the pad puts
-// the 64 lanes' slice chains in distinct banks) and return
+// One wave: stage the row src[0..D) in LDS (NormRow) and return
 //   r = 1 / sqrt(S / D + eps),  S = sum_d src[d]^2
 // in the canonical order: each square rounded to float, lane s adds the
 // squares of slice s (64 indices) in a sequential chain from +0.0f, and the
 // slice sums are combined by the zero-padded pairwise tree p[l] += p[l + st]
 // (the router's order); IEEE division and square root. The row stays in LDS
-// for the caller; every lane of the wave must call it, and gets r.
+// for the caller and, where it moves in pieces (NormRow::pieces), piece lane + 64 i
+// in v[i]; every lane of the wave must call it, and gets r.
 template <typename A>
-__device__ __forceinline__ float wave_rms_factor(const A* __restrict__ src, int D, float eps, float* row) {
+__device__ __forceinline__ float wave_rms_factor(const A* __restrict__ src, int D, float eps, A* row,
+                                                 uint4 (&v)[NormRow<A>::kPieces]) {
 #pragma clang fp contract(off)
+  using R = NormRow<A>;
   const int lane = threadIdx.x & 63;
   const int NS = (D + kRouterSlice - 1) / kRouterSlice;
   int P = 1;
   while (P < NS) P <<= 1;
-  // loads in batches of kNormBatch per lane, all issued before their LDS
-  // writes (addresses clamped into the row, so no load sits behind a branch)
-  for (int base = 0; base < D; base += 64 * kNormBatch) {
-    float v[kNormBatch];
+  const bool pieces = R::pieces(src, D);
+  if (pieces) {
+    const int n = D / R::kPiece;
 #pragma unroll
-    for (int j = 0; j < kNormBatch; ++j) v[j] = Act<A>::load(src, min(base + 64 * j + lane, D - 1));
-#pragma unroll
-    for (int j = 0; j < kNormBatch; ++j) {
-      const int d = base + 64 * j + lane;
-      if (d < D) row[(d >> 6) * (kRouterSlice + 1) + (d & 63)] = v[j];
+    for (int i = 0; i < R::kPieces; ++i) {
+      v[i] = uint4{0u, 0u, 0u, 0u};
+      if (lane + 64 * i < n) v[i] = reinterpret_cast<const uint4*>(src)[lane + 64 * i];
     }
+#pragma unroll
+    for (int i = 0; i < R::kPieces; ++i)
+      if (lane + 64 * i < n) *reinterpret_cast<uint4*>(row + R::at((lane + 64 * i) * R::kPiece)) = v[i];
+  } else {
+    for (int d = lane; d < D; d += 64) row[R::at(d)] = src[d];
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   float acc = 0.0f;
   if (lane < NS) {
-    const float* sl = row + lane * (kRouterSlice + 1);
-    const int n = min(kRouterSlice, D - lane * kRouterSlice);
-    for (int i = 0; i < n; ++i) {
-      const float sq = sl[i] * sl[i];
-      acc = acc + sq;
+    const A* sl = row + lane * R::kSlice;
+    if (pieces) {
+      // the slice's reads are all in flight before the chain starts
+      uint4 p[kRouterSlice / R::kPiece];
+#pragma unroll
+      for (int i = 0; i < kRouterSlice / R::kPiece; ++i) p[i] = reinterpret_cast<const uint4*>(sl)[i];
+#pragma unroll
+      for (int i = 0; i < kRouterSlice / R::kPiece; ++i) {
+        float f[R::kPiece];
+        R::unpack(p[i], f);
+#pragma unroll
+        for (int j = 0; j < R::kPiece; ++j) {
+          const float sq = f[j] * f[j];
+          acc = acc + sq;
+        }
+      }
+    } else {
+      const int n = min(kRouterSlice, D - lane * kRouterSlice);
+      for (int i = 0; i < n; ++i) {
+        const float x = Act<A>::load(sl, i);
+        const float sq = x * x;
+        acc = acc + sq;
+      }
     }
   }
   for (int st = 1; st < P; st <<= 1) {

@@ -309,17 +309,19 @@ __global__ __launch_bounds__(256) void k_route_slices(int T, int D, int E, int P
   __shared__ float xs[4][kRouterSlice][TB];
   __shared__ float red[2][TB * EPL][64];
   __shared__ float rfac[TB];
-  extern __shared__ float nrow[];  // with nm.scale: TB staged rows, norm_row_floats(D) each
+  extern __shared__ __attribute__((aligned(16))) uint8_t nrow[];  // with nm.scale: TB staged rows (NormRow)
   const int g = blockIdx.x, t0 = blockIdx.y * TB;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int s = 4 * g + w;
   const int d0 = s * kRouterSlice;
-  const int NRF = norm_row_floats(D);
+  const size_t NRB = NormRow<A>::bytes(D);
   if (nm.scale) {
     // x is the residual stream h: wave tt reduces row t0 + tt (the canonical
     // rms_norm order); the slices are normalised below
     if (w < TB && t0 + w < T) {
-      const float r = wave_rms_factor(x + (int64_t)(t0 + w) * D, D, nm.eps, nrow + w * NRF);
+      uint4 held[NormRow<A>::kPieces];
+      const float r =
+          wave_rms_factor(x + (int64_t)(t0 + w) * D, D, nm.eps, reinterpret_cast<A*>(nrow + w * NRB), held);
       if (lane == 0) rfac[w] = r;
     }
     __syncthreads();
@@ -333,7 +335,7 @@ __global__ __launch_bounds__(256) void k_route_slices(int T, int D, int E, int P
         // the block's input h2 = round_act((h * r) * scale): staged here and
         // written out for the expert kernels (each block writes its slices)
         const float sc = load_scale(nm.scale, nm.scale_bf16, d);
-        v = rms_apply<A>(nrow[tt * NRF + (d >> 6) * (kRouterSlice + 1) + (d & 63)], rfac[tt], sc);
+        v = rms_apply<A>(Act<A>::load(reinterpret_cast<const A*>(nrow + tt * NRB), NormRow<A>::at(d)), rfac[tt], sc);
         Act<A>::store(reinterpret_cast<A*>(nm.h2), (int64_t)(t0 + tt) * D + d, v);
       } else {
         v = Act<A>::load(x, (int64_t)(t0 + tt) * D + d);
@@ -1025,7 +1027,7 @@ static void launch_slices(const kmoe_desc& d, const SplitShape& sh, const void* 
   const int T = (int)d.tokens, D = (int)d.hidden, E = (int)d.num_experts;
   const int scale_bf16 = (r.dtype == KMOE_DTYPE_I8 && r.scale_dtype == KMOE_DTYPE_BF16) ? 1 : 0;
   const int scale_pc = (r.dtype == KMOE_DTYPE_I8 && r.scale_kind == KMOE_SCALE_CHANNEL) ? 1 : 0;
-  const size_t lds = nm.scale ? (size_t)TB * norm_row_floats(D) * sizeof(float) : 0;
+  const size_t lds = nm.scale ? (size_t)TB * NormRow<A>::bytes(D) : 0;
   hipLaunchKernelGGL((k_route_slices<A, RT, EPL, TB>), dim3(sh.Q, (T + TB - 1) / TB), dim3(256), lds, st, T, D, E,
                      sh.P, sh.Q, reinterpret_cast<const A*>(x), r.values, r.scale, scale_bf16, scale_pc, part, nm);
 }

@@ -1450,6 +1450,10 @@ __global__ __launch_bounds__(256) void k_combine8(int T, int K, int D, const A* 
   const int t = blockIdx.y;
   const int n0 = (blockIdx.x * blockDim.x + threadIdx.x) * 8;
   if (n0 >= D) return;
+  // the residual depends on nothing: requested before the selections, whose y rows
+  // are a second round trip (the T = 7 block call 61.5 -> 60.0 us)
+  float r[8];
+  if (res) Vec8<A>::load(res + (int64_t)t * D + n0, r);
   float acc[8];
 #pragma unroll
   for (int v = 0; v < 8; ++v) acc[v] = 0.0f;
@@ -1475,8 +1479,6 @@ __global__ __launch_bounds__(256) void k_combine8(int T, int K, int D, const A* 
   }
   if (res) {
     // the block's output is rounded to the activation dtype, then added to h
-    float r[8];
-    Vec8<A>::load(res + (int64_t)t * D + n0, r);
 #pragma unroll
     for (int v = 0; v < 8; ++v) acc[v] = r[v] + Act<A>::round(acc[v]);
   }
@@ -1550,6 +1552,9 @@ __global__ __launch_bounds__(1024) void k_down_combine(int T, int K, int TPB, in
       cw[j] = topk_w[a0 + (tid >> 4) * K + j];
     }
   }
+  // and its residual
+  const int64_t ro = (int64_t)(t0 + (tid >> 4)) * D + dt * 16 + (tid & 15);
+  const uint16_t rv = comb && res ? res[ro] : (uint16_t)0;
   const int p = m < nt * K ? inv[a0 + m] : -1;
   if (p >= 0) {
     const int e = topk_idx[a0 + m];
@@ -1625,9 +1630,8 @@ __global__ __launch_bounds__(1024) void k_down_combine(int T, int K, int TPB, in
         acc = combine_term<uint16_t, SCATTER>(acc, cw[j], round_bf16(v));
       }
     }
-    const int64_t o = (int64_t)(t0 + t) * D + dt * 16 + col;
-    if (res) acc = bf16_bits_to_f32(res[o]) + round_bf16(acc);
-    out[o] = f32_to_bf16_bits(acc);
+    if (res) acc = bf16_bits_to_f32(rv) + round_bf16(acc);
+    out[ro] = f32_to_bf16_bits(acc);
   }
 }
 

@@ -311,14 +311,16 @@ static __device__ void dispatch_chunk(int T, int E, int K, int b, int nblk, cons
 
 // The same dispatch by one wave with no barrier, for a call with at most 8
 // assignments (one token) and 256 experts (every thread may call it; wave 0
-// works). sel holds the T*K row-major selections (LDS or global, read by all
-// lanes at once). Assignment m = lane: its position is the number of
-// assignments with a smaller expert plus the earlier ones with the same expert
-// (the stable sort); an expert's count and offset come from one pass over the
-// selections. It is correct up to 64 assignments, but its serial passes cost
-// more than dispatch_chunk's barriers from 16 assignments on (T=1 decode
-// layer 24.4 -> 23.7 us; T=4 and T=8 2 and 5 us slower).
-__device__ __forceinline__ bool dispatch_fits_wave(int M, int E) { return M <= 8 && E <= 256; }
+// works). sel holds the T*K row-major selections (LDS or global). Assignment m =
+// lane: its position is the number of assignments with a smaller expert plus the
+// earlier ones with the same expert (the stable sort); an expert's count and
+// offset come from one pass over the selections, which sit in scalar registers
+// (read by every lane from LDS, one after the other, with the combine's residual read
+// last, the T = 1 block call took 24.7 us instead of 24.15). Its serial passes cost
+// more than dispatch_chunk's barriers from 16 assignments on (T=1 decode layer
+// 24.4 -> 23.7 us; T=4 and T=8 2 and 5 us slower).
+constexpr int kDispatchWaveMax = 8;
+__device__ __forceinline__ bool dispatch_fits_wave(int M, int E) { return M <= kDispatchWaveMax && E <= 256; }
 
 static __device__ void dispatch_wave(int T, int E, int K, const int32_t* sel, int32_t* __restrict__ group_sizes,
                                      int32_t* __restrict__ offsets, int32_t* __restrict__ active,
@@ -328,18 +330,21 @@ static __device__ void dispatch_wave(int T, int E, int K, const int32_t* sel, in
   const int lane = threadIdx.x & 63;
   const int M = T * K;
   const int em = lane < M ? sel[lane] : -1;
+  int s[kDispatchWaveMax];  // selection i, -1 past the last
+#pragma unroll
+  for (int i = 0; i < kDispatchWaveMax; ++i) s[i] = __builtin_amdgcn_readlane(em, i);
   int below = 0, before = 0;
-  for (int i = 0; i < M; ++i) {
-    const int ei = sel[i];
-    below += ei < em;
-    before += ei == em && i < lane;
+#pragma unroll
+  for (int i = 0; i < kDispatchWaveMax; ++i) {
+    below += i < M && s[i] < em;
+    before += s[i] == em && i < lane;
   }
   // an assignment that is its expert's first: its index among the active experts
   const bool first = lane < M && before == 0;
   const unsigned long long firsts = __ballot(first);
   int rank = 0;
-  for (int i = 0; i < M; ++i)
-    if ((firsts >> i) & 1ull) rank += sel[i] < em;
+#pragma unroll
+  for (int i = 0; i < kDispatchWaveMax; ++i) rank += ((firsts >> i) & 1ull) && s[i] < em;
   if (lane < M) {
     const int p = below + before;
     sorted_token[p] = lane / K;
@@ -349,10 +354,10 @@ static __device__ void dispatch_wave(int T, int E, int K, const int32_t* sel, in
   }
   for (int e = lane; e < E; e += 64) {
     int cnt = 0, less = 0;
-    for (int i = 0; i < M; ++i) {
-      const int ei = sel[i];
-      cnt += ei == e;
-      less += ei < e;
+#pragma unroll
+    for (int i = 0; i < kDispatchWaveMax; ++i) {
+      cnt += s[i] == e;
+      less += i < M && s[i] < e;
     }
     group_sizes[e] = cnt;
     offsets[e] = less;

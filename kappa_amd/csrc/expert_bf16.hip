@@ -508,8 +508,6 @@ hipError_t w16_stages(const kmoe_desc& d, int family, int stages, const uint16_t
   return hipSuccess;
 }
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
 }  // namespace
 
 bool expert_w16_fits(const kmoe_desc& d, int stages, const void* x, const kmoe_weight* gate, const kmoe_weight* up,

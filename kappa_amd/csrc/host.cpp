@@ -69,8 +69,21 @@ bool route_mfma_preferred(const kmoe_desc& d, const kmoe_weight& router) {
   return route_mfma_fits(d, router) && d.tokens >= kRouteOwnScratchTokens;
 }
 
-int64_t route_mfma_place(const kmoe_desc& d, const kmoe_weight& router, const Workspace& w) {
-  if (!route_mfma_fits(d, router)) return -1;
+// Just above 510 tokens the all-VALU router's blocks of two tokens fill the chip's CUs
+// once, and it beats the two-phase router's latency: whole layers, all-VALU against
+// two-phase, 30B-A3B T = 512 / 560 / 600 / 640 159 / 166 / 168.6 / 170.6 against 165 / 169 /
+// 169.7 / 169.7 us; D = 2560, E = 64, T = 512 / 576 / 640 154 / 162 / 170 against 159 / 165 /
+// 169; 235B-A22B T = 511 / 576 484 / 508 against 493 / 503; E = 256, T = 512 / 576 260 / 280
+// against 262 / 266. On either side (blocks of one token, or a second round) it is
+// 5 to 30 us behind, and so with 32 experts (T = 512 127 against 117).
+static bool route_one_round(const kmoe_desc& d) {
+  const int64_t blocks = (d.tokens + 1) / 2;
+  const int64_t most = d.hidden <= 2560 && d.num_experts <= 128 ? 300 : 256;
+  return d.num_experts >= 64 && blocks >= 256 && blocks <= most;
+}
+
+int64_t route_mfma_place(const kmoe_desc& d, const void* x, const kmoe_weight& router, const Workspace& w) {
+  if (!route_mfma_fits(d, router) || !aligned16(x) || !aligned16(router.values) || route_one_round(d)) return -1;
   if (route_mfma_preferred(d, router)) return (int64_t)w.route_part;
   return w.route_part - w.h_sorted >= route_mfma_scratch_bytes(d) ? (int64_t)w.h_sorted : -1;
 }

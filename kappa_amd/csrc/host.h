@@ -100,6 +100,8 @@ inline int enum_value(const En& e) {
   return v;
 }
 
+inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 // Split router: group partials per token and expert, and their floats.
 int route_split_groups(const kmoe_desc& d);
 size_t route_split_part_floats(const kmoe_desc& d);
@@ -156,9 +158,10 @@ struct Workspace {
 bool down_planes_fits(const kmoe_desc& d);
 Workspace layout(const kmoe_desc& d, bool block);
 // Workspace offset of the two-phase router's scratch for this call; -1 where the
-// all-VALU router runs instead (the shape does not fit, or h_sorted and y_sorted
-// are smaller than the scratch).
-int64_t route_mfma_place(const kmoe_desc& d, const kmoe_weight& router, const Workspace& w);
+// all-VALU router runs instead (the shape does not fit, x or the router is not
+// 16-byte aligned, h_sorted and y_sorted are smaller than the scratch, or it is the
+// faster one: just above 510 tokens).
+int64_t route_mfma_place(const kmoe_desc& d, const void* x, const kmoe_weight& router, const Workspace& w);
 
 // --- argument checks ---------------------------------------------------------
 kmoe_status check_desc(const kmoe_desc* d);

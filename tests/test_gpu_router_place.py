@@ -22,11 +22,12 @@ def dev():
 
 # the first size of the two-phase router, with its scratch in the expert buffers; a
 # reduction of forty slices; expert buffers smaller than the scratch and a hidden size
-# it does not take (the all-VALU router); two halves of 128 experts, the second partial
+# it does not take (the all-VALU router); two halves of 128 experts, the second partial;
+# the edges of the sizes just above 510 tokens that the all-VALU router keeps
 @pytest.mark.parametrize(
     "T,D,E,K,I",
     [(241, 512, 32, 4, 128), (300, 2560, 64, 6, 64), (300, 512, 256, 1, 64), (260, 640, 32, 2, 64),
-     (500, 768, 176, 8, 64)],
+     (500, 768, 176, 8, 64), (511, 512, 64, 4, 64), (601, 512, 64, 4, 64)],
 )  # fmt: skip
 def test_layer_routing_above_the_split_router(dev, T, D, E, K, I):
     from kappa_amd.qwen3 import quantize_weight
@@ -44,6 +45,26 @@ def test_layer_routing_above_the_split_router(dev, T, D, E, K, I):
     assert np.all(np.abs(w.float().cpu().numpy() - ow) <= 2.0**-8 * np.abs(ow))
 
 
+def _shifted(t):
+    """The same values one element into a storage: not 16-byte aligned."""
+    v = torch.zeros(t.numel() + 8, dtype=t.dtype, device=t.device)[1 : 1 + t.numel()].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+def test_route_off_alignment(dev):
+    """Rows that are not 16-byte aligned take the all-VALU router: the same selections."""
+    from kappa_amd.qwen3 import moe_stages
+
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = torch.randn(300, 1024, generator=g, device=dev).to(torch.bfloat16)
+    router = (torch.randn(1024, 64, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    want = moe_stages.route(x, router, num_experts=64, k=4, logits=False)
+    got = moe_stages.route(_shifted(x), router, num_experts=64, k=4, logits=False)
+    for n in ("idx", "w", "hist"):
+        assert torch.equal(got[n], want[n]), n
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("which", ["x", "scale"])
 def test_rms_norm_off_alignment(dev, dtype, which):
@@ -54,11 +75,5 @@ def test_rms_norm_off_alignment(dev, dtype, which):
     x = torch.randn(9, 2048, generator=g, device=dev).to(dtype)
     s = torch.randn(2048, generator=g, device=dev).to(dtype)
     want = rms_norm(x, s)
-
-    def shifted(t):
-        v = torch.zeros(t.numel() + 8, dtype=t.dtype, device=dev)[1 : 1 + t.numel()].view(t.shape)
-        v.copy_(t)
-        return v
-
-    got = rms_norm(shifted(x) if which == "x" else x, shifted(s) if which == "scale" else s)
+    got = rms_norm(_shifted(x) if which == "x" else x, _shifted(s) if which == "scale" else s)
     assert torch.equal(got, want)

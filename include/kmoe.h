@@ -244,7 +244,10 @@ kmoe_status kmoe_dispatch(const kmoe_desc* desc, const int32_t* topk_idx, const 
 /* SwiGLU experts over the sorted rows (kappa/qwen3/ffn_moe.py:99-102,
  * 149-152, 207-210): y_sorted [T*K, D] in x.dtype; h_sorted [T*K, I] in x.dtype,
  * except for the RAGGED chain with bf16 activations, whose f32 h is stored as
- * [T*K, 2I] bf16: per row hi = bf16(h) in [0, I) and lo = bf16(h - hi) in [I, 2I). */
+ * [T*K, 2I] bf16: per row hi = bf16(h) in [0, I) and lo = bf16(h - hi) in [I, 2I).
+ * The row arrays are kmoe_dispatch's. Every row is written, whatever the capacity,
+ * but with packed experts: those leave the rows at or past desc->expert_capacity of
+ * each expert as they were. */
 kmoe_status kmoe_expert_ffn(const kmoe_desc* desc, const void* x, const int32_t* offsets, const int32_t* active,
                             const int32_t* sorted_token, const int32_t* sorted_expert, const kmoe_weight* gate,
                             const kmoe_weight* up, const kmoe_weight* down, const kmoe_packed_experts* packed,

@@ -32,17 +32,23 @@ kmoe_status device_status() {
     if (_e != hipSuccess) return hip_fail(_e, what);  \
   } while (0)
 
-kmoe_status expert_stage(const kmoe_desc& d, int stages, const void* x, const int32_t* offsets, const int32_t* active,
-                         const int32_t* sorted_token, const int32_t* sorted_expert, const kmoe_weight* gate,
-                         const kmoe_weight* up, const kmoe_weight* down, const kmoe_packed_experts* packed,
-                         void* h_sorted, void* y_sorted, hipStream_t st, float* h_scale = nullptr) {
+constexpr int kEveryRow = 0x7fffffff;
+
+// cap: the rows per expert that plain bf16 experts compute. The whole call's combine
+// skips the others (inv < 0); the stage calls give every row of the sorted list, as
+// the layout-native kernels do (packed experts keep the desc's capacity in both).
+kmoe_status expert_stage(const kmoe_desc& d, int cap, int stages, const void* x, const int32_t* offsets,
+                         const int32_t* active, const int32_t* sorted_token, const int32_t* sorted_expert,
+                         const kmoe_weight* gate, const kmoe_weight* up, const kmoe_weight* down,
+                         const kmoe_packed_experts* packed, void* h_sorted, void* y_sorted, hipStream_t st,
+                         float* h_scale = nullptr) {
   hipError_t e;
   if (packed_ok(d, packed)) {
     e = launch_expert_packed(d, chain_of(d), family_of(d), stages, x, offsets, active, sorted_token, *packed,
                              h_sorted, y_sorted, st, h_scale);
   } else if (expert_w16_fits(d, stages, x, gate, up, down, h_sorted, y_sorted)) {
     e = launch_expert_w16(d, chain_of(d), family_of(d), stages, x, offsets, active, sorted_token, gate, up, down,
-                          h_sorted, y_sorted, st);
+                          h_sorted, y_sorted, cap, st);
   } else {
     e = launch_expert_generic(d, chain_of(d), stages, x, sorted_token, sorted_expert, gate, up, down, h_sorted,
                               y_sorted, st);
@@ -111,8 +117,8 @@ kmoe_status kmoe_expert_ffn(const kmoe_desc* desc, const void* x, const int32_t*
                            h_sorted, y_sorted));
   KMOE_TRY(device_status());
   if (desc->tokens == 0) return KMOE_OK;
-  return expert_stage(*desc, both, x, offsets, active, sorted_token, sorted_expert, gate, up, down, packed, h_sorted,
-                      y_sorted, (hipStream_t)stream);
+  return expert_stage(*desc, kEveryRow, both, x, offsets, active, sorted_token, sorted_expert, gate, up, down, packed,
+                      h_sorted, y_sorted, (hipStream_t)stream);
 }
 
 kmoe_status kmoe_expert_gate_up(const kmoe_desc* desc, const void* x, const int32_t* offsets, const int32_t* active,
@@ -123,8 +129,8 @@ kmoe_status kmoe_expert_gate_up(const kmoe_desc* desc, const void* x, const int3
                            packed, h_sorted, nullptr));
   KMOE_TRY(device_status());
   if (desc->tokens == 0) return KMOE_OK;
-  return expert_stage(*desc, kStageGateUp, x, offsets, active, sorted_token, sorted_expert, gate, up, nullptr, packed,
-                      h_sorted, nullptr, (hipStream_t)stream);
+  return expert_stage(*desc, kEveryRow, kStageGateUp, x, offsets, active, sorted_token, sorted_expert, gate, up,
+                      nullptr, packed, h_sorted, nullptr, (hipStream_t)stream);
 }
 
 kmoe_status kmoe_expert_down(const kmoe_desc* desc, const void* h_sorted, const int32_t* offsets,
@@ -134,8 +140,8 @@ kmoe_status kmoe_expert_down(const kmoe_desc* desc, const void* h_sorted, const 
                            down, packed, h_sorted, y_sorted));
   KMOE_TRY(device_status());
   if (desc->tokens == 0) return KMOE_OK;
-  return expert_stage(*desc, kStageDown, nullptr, offsets, active, nullptr, sorted_expert, nullptr, nullptr, down,
-                      packed, const_cast<void*>(h_sorted), y_sorted, (hipStream_t)stream);
+  return expert_stage(*desc, kEveryRow, kStageDown, nullptr, offsets, active, nullptr, sorted_expert, nullptr, nullptr,
+                      down, packed, const_cast<void*>(h_sorted), y_sorted, (hipStream_t)stream);
 }
 
 kmoe_status kmoe_combine(const kmoe_desc* desc, const void* y_sorted, const int32_t* inv, const float* topk_w,
@@ -249,15 +255,15 @@ kmoe_status forward_general(const kmoe_desc* desc, const void* x, const void* xi
   if (packed_ok(*desc, packed) && family_of(*desc) == kFamilyDecode &&
       down_combine_fits(*desc, chain)) {
     // at most 32 assignments: the down projection and the combine in one kernel
-    KMOE_TRY(expert_stage(*desc, kStageGateUp, xin, off, act, stok, sexp, gate, up, down, packed, hs, ys,
-                          st));
+    KMOE_TRY(expert_stage(*desc, capacity_of(*desc), kStageGateUp, xin, off, act, stok, sexp, gate, up, down, packed,
+                          hs, ys, st));
     KMOE_HIP(launch_down_combine(*desc, chain, scatter, hs, tidx, inv, tw, *packed, out, st, res),
              "down+combine kernel");
   } else {
     // with down_planes_fits the workspace's h rows become int8 planes, their
     // scales in w.h_scale
     float* hscale = down_planes_fits(*desc) ? reinterpret_cast<float*>(base + w.h_scale) : nullptr;
-    KMOE_TRY(expert_stage(*desc, kStageGateUp | kStageDown, xin, off, act, stok, sexp, gate,
+    KMOE_TRY(expert_stage(*desc, capacity_of(*desc), kStageGateUp | kStageDown, xin, off, act, stok, sexp, gate,
                           up, down, packed, hs, ys, st, hscale));
     KMOE_HIP(launch_combine(*desc, scatter, ys, inv, tw, out, st, res), "combine kernel");
   }

@@ -471,13 +471,12 @@ namespace {
 template <int CH>
 hipError_t w16_stages(const kmoe_desc& d, int family, int stages, const uint16_t* x, const int32_t* offsets,
                       const int32_t* active, const int32_t* sorted_token, const uint16_t* wg, const uint16_t* wu,
-                      const uint16_t* wd, uint16_t* hb, uint16_t* yb, hipStream_t st) {
+                      const uint16_t* wd, uint16_t* hb, uint16_t* yb, int cap, hipStream_t st) {
   const int T = (int)d.tokens, D = (int)d.hidden, E = (int)d.num_experts, K = (int)d.top_k,
             I = (int)d.intermediate;
   const int M = T * K;
   const int slots = M < E ? M : E;
-  const int cap = capacity_of(d);
-    // the GEMV form up to 64 tokens, as for int8 experts: whole 30B-A3B layers, GEMV
+  // the GEMV form up to 64 tokens, as for int8 experts: whole 30B-A3B layers, GEMV
   // against GEMM, T = 1 / 4 / 16 / 64 41 / 76 / 157 / 228 against 75 / 94 / 187 /
   // 255 us. Above 64 tokens it still leads on that shape (T = 65 / 100 234 / 247
   // against 259 / 262 us) and trails on wider or fewer experts (235B-A22B T = 100
@@ -527,16 +526,16 @@ bool expert_w16_fits(const kmoe_desc& d, int stages, const void* x, const kmoe_w
 hipError_t launch_expert_w16(const kmoe_desc& d, int chain, int family, int stages, const void* x,
                              const int32_t* offsets, const int32_t* active, const int32_t* sorted_token,
                              const kmoe_weight* gate, const kmoe_weight* up, const kmoe_weight* down, void* h_sorted,
-                             void* y_sorted, hipStream_t st) {
+                             void* y_sorted, int cap, hipStream_t st) {
   auto v = [](const kmoe_weight* w) { return w ? reinterpret_cast<const uint16_t*>(w->values) : nullptr; };
   const uint16_t* xb = reinterpret_cast<const uint16_t*>(x);
   uint16_t* hb = reinterpret_cast<uint16_t*>(h_sorted);
   uint16_t* yb = reinterpret_cast<uint16_t*>(y_sorted);
   if (chain == kChainF32)
     return w16_stages<kChainF32>(d, family, stages, xb, offsets, active, sorted_token, v(gate), v(up), v(down), hb, yb,
-                                 st);
+                                 cap, st);
   return w16_stages<kChainAct>(d, family, stages, xb, offsets, active, sorted_token, v(gate), v(up), v(down), hb, yb,
-                               st);
+                               cap, st);
 }
 
 }  // namespace kmoe_host

@@ -72,14 +72,13 @@ hipError_t launch_expert_generic(const kmoe_desc& d, int chain, int stages, cons
 // Plain bf16 experts in the reference layout on MFMA (expert_bf16.hip): whether
 // a call's stages can take them (bf16 activations and weights, D and I multiples
 // of 64, 16-byte aligned buffers, 32-bit load offsets), and the launch. Buffers
-// as the layout-native kernels'; only each expert's first capacity rows are
-// computed.
+// as the layout-native kernels'; only each expert's first cap rows are computed.
 bool expert_w16_fits(const kmoe_desc& d, int stages, const void* x, const kmoe_weight* gate, const kmoe_weight* up,
                      const kmoe_weight* down, const void* h_sorted, const void* y_sorted);
 hipError_t launch_expert_w16(const kmoe_desc& d, int chain, int family, int stages, const void* x,
                              const int32_t* offsets, const int32_t* active, const int32_t* sorted_token,
                              const kmoe_weight* gate, const kmoe_weight* up, const kmoe_weight* down, void* h_sorted,
-                             void* y_sorted, hipStream_t st);
+                             void* y_sorted, int cap, hipStream_t st);
 // out = the terms round(w * y_sorted[inv]) summed in f32 and rounded once
 // (scatter = false) or added into a rounded running sum (scatter = true)
 // [+ residual res, rounded again], res may be NULL

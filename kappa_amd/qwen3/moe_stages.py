@@ -118,8 +118,9 @@ def expert_ffn(
     lo = bf16(h - hi) of its f32 h.
 
     ``layout_native=True`` runs the kernels that read the reference layout
-    directly (one fmaf chain per output) instead of the packed MFMA kernels;
-    ``kernels`` picks the packed family (``_lib.KERNELS_*``).
+    directly instead of the packed ones: MFMA for bf16 weights whose widths are
+    multiples of 64, else one fmaf chain per output. ``kernels`` picks the MFMA
+    family (``_lib.KERNELS_*``).
     ``capacity > 0``: the packed kernels compute only each expert's first
     ``capacity`` rows (the others are left as they were)."""
     T, D = x_flat.shape

@@ -86,3 +86,21 @@ def test_bf16_weights_off_alignment(dev, T):
         np.testing.assert_array_equal(idx.cpu().numpy(), ref["idx"])
         got = out.reshape(T, D).float().cpu().numpy()
         assert np.abs(got - ref["out"]).max() <= 2e-2 and mean_rel(got, ref["out"]) <= 1e-3, which
+
+
+@pytest.mark.parametrize("T", [5, 100])
+def test_bf16_stage_writes_every_row(dev, T):
+    """The stage call computes the rows past an expert's capacity too (the whole call's
+    combine is what drops them)."""
+    from kappa_amd.qwen3 import moe_stages
+
+    xn, rn, *wn = _layer(T + 1, T)
+    x, router, *ws = (_dev_bf16(a, dev) for a in (xn, rn, *wn))
+    r = moe_stages.route(x, router, num_experts=E, k=K)
+    d = moe_stages.dispatch(r["idx"], r["hist"], num_experts=E, capacity=1)
+    assert bool((d["group_sizes"] > 1).any())
+    _, y = moe_stages.expert_ffn(x, d, *ws, k=K, impl="fixed_capacity", capacity=1)
+    _, ref = oracle.expert_ffn(xn, d["offsets"].cpu().numpy(), d["sorted_token"].cpu().numpy(), *wn, True,
+                               impl="fixed_capacity")  # fmt: skip
+    got = y.float().cpu().numpy()
+    assert np.abs(got - ref).max() <= 2e-2 and mean_rel(got, ref) <= 1e-3

@@ -155,7 +155,9 @@ const char* kmoe_last_error(void);
 kmoe_status kmoe_device_check(void);
 
 /* --- sizes ---------------------------------------------------------------- */
-/* Bytes of device workspace kmoe_forward needs for this problem. */
+/* Bytes of device workspace kmoe_forward and kmoe_forward_block need for this problem.
+ * Never less than for fewer tokens of the same layer: a workspace sized for the
+ * largest call serves every smaller one. */
 kmoe_status kmoe_workspace_bytes(const kmoe_desc* desc, size_t* bytes);
 /* Sizes of the packed expert buffers (requires D % 64 == 0, I % 64 == 0). */
 kmoe_status kmoe_prepack_bytes(const kmoe_desc* desc, kmoe_packed_sizes* sizes);
@@ -230,7 +232,10 @@ kmoe_status kmoe_route(const kmoe_desc* desc, const void* x, const kmoe_weight* 
                        void* scratch, size_t scratch_bytes, int32_t* topk_idx, float* topk_w, int32_t* block_hist,
                        void* stream);
 /* Bytes of scratch the two-phase form of kmoe_route needs (the router
- * transposed to bf16, its column norms' partial sums and the partial logits). */
+ * transposed to bf16, its column norms' partial sums and the partial logits); never
+ * less than for fewer tokens. A scratch below the first two parts
+ * (2 E D + 4 E ceil(D / 256) bytes, the first rounded up to 256) is refused; between
+ * the two, and wherever the two-phase form does not apply, the call uses none of it. */
 kmoe_status kmoe_route_scratch_bytes(const kmoe_desc* desc, size_t* bytes);
 
 /* Stable sort of assignments by expert (kappa/qwen3/ffn_moe.py:189-200, 212):

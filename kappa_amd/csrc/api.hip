@@ -88,7 +88,8 @@ kmoe_status kmoe_route(const kmoe_desc* desc, const void* x, const kmoe_weight* 
   KMOE_TRY(device_status());
   if (desc->tokens == 0) return KMOE_OK;
   hipError_t e =
-      !logits && scratch && route_mfma_fits(*desc, *router) && aligned16(x) && aligned16(router->values)
+      !logits && scratch && route_mfma_fits(*desc, *router) && aligned16(x) && aligned16(router->values) &&
+              scratch_bytes >= route_mfma_scratch_bytes(*desc)
           ? launch_route_mfma(*desc, x, *router, scratch, topk_idx, topk_w, block_hist, (hipStream_t)stream)
           : launch_route(*desc, x, *router, logits, topk_idx, topk_w, block_hist, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "route kernels");

@@ -59,10 +59,14 @@ size_t route_split_part_floats(const kmoe_desc& d) {
   return (size_t)d.tokens * route_split_groups(d) * d.num_experts;
 }
 
-bool route_mfma_fits(const kmoe_desc& d, const kmoe_weight& router) {
+static bool route_mfma_shape(const kmoe_desc& d) {
   const int64_t D = d.hidden;
-  return enum_value(d.act_dtype) == KMOE_DTYPE_BF16 && enum_value(router.dtype) == KMOE_DTYPE_BF16 && D % 256 == 0 &&
-         D >= 512 && D <= 4096 && d.num_experts % 16 == 0 && d.num_experts <= 256;
+  return enum_value(d.act_dtype) == KMOE_DTYPE_BF16 && D % 256 == 0 && D >= 512 && D <= 4096 &&
+         d.num_experts % 16 == 0 && d.num_experts <= 256;
+}
+
+bool route_mfma_fits(const kmoe_desc& d, const kmoe_weight& router) {
+  return route_mfma_shape(d) && enum_value(router.dtype) == KMOE_DTYPE_BF16;
 }
 
 bool route_mfma_preferred(const kmoe_desc& d, const kmoe_weight& router) {
@@ -88,23 +92,40 @@ int64_t route_mfma_place(const kmoe_desc& d, const void* x, const kmoe_weight& r
   return w.route_part - w.h_sorted >= route_mfma_scratch_bytes(d) ? (int64_t)w.h_sorted : -1;
 }
 
+constexpr int64_t kRouteTiles = 256;  // blocks of the logits kernel, splits times 64-token tiles
+
 int route_mfma_splits(const kmoe_desc& d) {
   // blocks of 64 tokens; splits while they still fit the chip's CUs once
   const int64_t tiles = (d.tokens + 63) / 64;
   int ks = kmoe::kRouteMaxSplits;
-  while (ks > 1 && tiles * ks > 256) ks >>= 1;
+  while (ks > 1 && tiles * ks > kRouteTiles) ks >>= 1;
   return ks;
 }
 
 size_t route_mfma_scratch_offsets(const kmoe_desc& d, int part) {
-  const size_t E = (size_t)d.num_experts, D = (size_t)d.hidden, KS = (size_t)route_mfma_splits(d);
+  const size_t E = (size_t)d.num_experts, D = (size_t)d.hidden, KS = kmoe::kRouteMaxSplits;
+  // splits * tokens is largest at this call's tokens or at the last size of any number of
+  // splits: 64 * kRouteTiles each time
+  const size_t own = (size_t)route_mfma_splits(d) * (size_t)d.tokens, first = KS * (size_t)d.tokens;
+  const size_t full = 64 * (size_t)kRouteTiles;
+  const size_t rows = own > full ? own : (first < full ? first : full);
   const size_t o1 = align_up(2 * E * D);
   const size_t o2 = align_up(o1 + 4 * KS * E);
-  const size_t o3 = o2 + 4 * KS * (size_t)d.tokens * E;
+  const size_t o3 = o2 + 4 * rows * E;
   return part == 1 ? o1 : (part == 2 ? o2 : (part == 3 ? o3 : 0));
 }
 
-size_t route_mfma_scratch_bytes(const kmoe_desc& d) { return route_mfma_scratch_offsets(d, 3); }
+size_t route_scratch_min_bytes(const kmoe_desc& d) {
+  const size_t E = (size_t)d.num_experts, D = (size_t)d.hidden;
+  return align_up(2 * E * D) + 4 * ((D + 255) / 256) * E;
+}
+
+size_t route_mfma_scratch_bytes(const kmoe_desc& d) {
+  const size_t least = route_scratch_min_bytes(d);
+  if (!route_mfma_shape(d)) return least;
+  const size_t all = route_mfma_scratch_offsets(d, 3);
+  return all > least ? all : least;
+}
 
 bool is_float(kmoe_dtype t) {
   const int v = enum_value(t);
@@ -224,7 +245,13 @@ Workspace layout(const kmoe_desc& d, bool block) {
                                                          : (T >= (size_t)kRouteOwnScratchTokens ? route_mfma_scratch_bytes(d) : 0));
   w.h_scale = take(down_planes_fits(d) ? 4 * M : 0);
   w.normed = take(block ? act * T * D : 0);  // rms_norm(h) for kmoe_forward_block
-  w.total = o;
+  w.end = w.total = o;
+  if (block && T > (size_t)kSplitRouterMaxTokens) {
+    kmoe_desc split = d;
+    split.tokens = kSplitRouterMaxTokens;
+    const size_t below = layout(split, true).end;
+    if (w.total < below) w.total = below;
+  }
   return w;
 }
 
@@ -359,9 +386,9 @@ kmoe_status validate_forward_block(const kmoe_desc* desc, const void* h, const v
     return fail(KMOE_ERR_INVALID_ARG, "kmoe_forward_block: h and out must be non-NULL");
   if (desc->tokens > 0 && out == h) return fail(KMOE_ERR_INVALID_ARG, "kmoe_forward_block: out must not alias h");
   *w = layout(*desc, true);
-  if (desc->tokens > 0 && (!workspace || workspace_bytes < w->total))
+  if (desc->tokens > 0 && (!workspace || workspace_bytes < w->end))
     return fail(KMOE_ERR_WORKSPACE_TOO_SMALL, "workspace of %zu bytes is smaller than the %zu required",
-                workspace_bytes, w->total);
+                workspace_bytes, w->end);
   return KMOE_OK;
 }
 
@@ -391,9 +418,9 @@ kmoe_status validate_route(const kmoe_desc* desc, const void* x, const kmoe_weig
   KMOE_TRY(check_desc(desc));
   KMOE_TRY(check_weight(router, "router"));
   if (!x || !topk_idx || !topk_w || !block_hist) return fail(KMOE_ERR_INVALID_ARG, "kmoe_route: NULL buffer");
-  if (scratch && scratch_bytes < route_mfma_scratch_bytes(*desc))
+  if (scratch && scratch_bytes < route_scratch_min_bytes(*desc))
     return fail(KMOE_ERR_WORKSPACE_TOO_SMALL, "kmoe_route: scratch of %zu bytes is smaller than the %zu required",
-                scratch_bytes, route_mfma_scratch_bytes(*desc));
+                scratch_bytes, route_scratch_min_bytes(*desc));
   return KMOE_OK;
 }
 

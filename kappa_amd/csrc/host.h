@@ -110,11 +110,17 @@ size_t route_split_part_floats(const kmoe_desc& d);
 // 4096, E % 16 == 0, E <= 256), the splits of its reduction over blocks (KS), and its
 // scratch: the router transposed to bf16 [E][8][D/64][8] (offset 0), the partial sums
 // of squares of its columns [KS][E] f32 (offset part 1) and the partial logits
-// [KS][T][E] f32 (part 2); part 3 is the total.
+// [KS][T][E] f32 (part 2); part 3 is the total. KS falls as T grows, so parts and total
+// are sized for the largest KS and KS * T of any call of up to T tokens: a scratch
+// (and a workspace) that serves T tokens serves every smaller call.
 bool route_mfma_fits(const kmoe_desc& d, const kmoe_weight& router);
 int route_mfma_splits(const kmoe_desc& d);
 size_t route_mfma_scratch_offsets(const kmoe_desc& d, int part);
 size_t route_mfma_scratch_bytes(const kmoe_desc& d);
+// What kmoe_route asks of a scratch whatever the token count and the router (the
+// transposed router and a norm per column and 256 hidden indices); with less than
+// route_mfma_scratch_bytes it runs the all-VALU router.
+size_t route_scratch_min_bytes(const kmoe_desc& d);
 // kmoe_forward routes with it above the split router's sizes. From this many tokens
 // the workspace holds a scratch for it (route_mfma_preferred); below, the scratch is in
 // the h_sorted and y_sorted buffers, which nothing uses before the expert
@@ -143,10 +149,13 @@ int family_of(const kmoe_desc& d);
 bool packed_ok(const kmoe_desc& d, const kmoe_packed_experts* p);
 
 // Byte offsets of the workspace buffers; block: also the normalised rows h2
-// that only kmoe_forward_block writes.
+// that only kmoe_forward_block writes. end: what the call itself needs; total: what is
+// asked of the caller. kmoe_workspace_bytes reports the block's total, which no smaller
+// call of the same layer exceeds: just above the split router's sizes, where its
+// partials are gone, it is the end at the largest of those.
 struct Workspace {
   size_t topk_idx, topk_w, hist, group_sizes, offsets, active, sorted_token, sorted_expert, inv, h_sorted,
-      y_sorted, route_part, h_scale, normed, total;
+      y_sorted, route_part, h_scale, normed, end, total;
 };
 // Whether the whole-block call's f32-chain down product takes h as int8 planes
 // (k_h_planes + the integer k_gemm): bf16 activations, the ragged program, at

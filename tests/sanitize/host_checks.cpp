@@ -371,6 +371,66 @@ static void layout_sweep() {
             }
 }
 
+// A caller sizes its buffers once, for its largest call: the reported sizes never
+// fall as the tokens grow, and every smaller call is accepted with them.
+static void sizes_never_fall() {
+  struct {
+    int64_t D, E, K, I;
+    kmoe_dtype act;
+    kmoe_impl impl;
+    int64_t thr;
+  } layers[] = {
+      {2048, 128, 8, 768, KMOE_DTYPE_BF16, KMOE_IMPL_RAGGED, 64},
+      {4096, 128, 8, 1536, KMOE_DTYPE_BF16, KMOE_IMPL_RAGGED, 0},
+      {2048, 256, 8, 768, KMOE_DTYPE_BF16, KMOE_IMPL_FIXED_CAPACITY, 0},
+      {2048, 32, 4, 960, KMOE_DTYPE_BF16, KMOE_IMPL_GATHER_EINSUM, 0},
+      {64, 1024, 1, 64, KMOE_DTYPE_BF16, KMOE_IMPL_RAGGED, 0},
+      {512, 256, 1, 64, KMOE_DTYPE_F32, KMOE_IMPL_RAGGED, 0},
+  };
+  const kmoe_weight fr = weight(P, KMOE_DTYPE_F32, nullptr, KMOE_DTYPE_F32, KMOE_SCALE_NONE);
+  const int32_t* I32 = reinterpret_cast<const int32_t*>(P);
+  const float* F32 = reinterpret_cast<const float*>(P);
+  for (auto& l : layers) {
+    size_t ws = 0, rs = 0, first_rs = 0;
+    bool ok = true;
+    for (int64_t T = 0; T <= 17000; ++T) {
+      const kmoe_desc d = desc(T, l.D, l.E, l.K, l.I, l.act, l.thr, l.impl == KMOE_IMPL_FIXED_CAPACITY ? 5 : 0, l.impl);
+      size_t n = 0, r = 0;
+      ok = ok && validate_workspace_bytes(&d, &n) == KMOE_OK && validate_route_scratch_bytes(&d, &r) == KMOE_OK;
+      if (n < ws || r < rs) {
+        ++g_fail;
+        fprintf(stderr, "sizes fall at T=%lld D=%lld E=%lld: workspace %zu after %zu, route scratch %zu after %zu\n",
+                (long long)T, (long long)l.D, (long long)l.E, n, ws, r, rs);
+        break;
+      }
+      ws = n, rs = r;
+      if (T == 0) first_rs = r;
+      // the call runs within what is reported, and the scratch holds its own parts
+      Workspace w;
+      ok = ok && (T == 0 || validate_forward(&d, P, &F, &F, &F, &F, nullptr, P, P, n, &w) == KMOE_OK);
+      ok = ok && (T == 0 || validate_forward_block(&d, P, P, KMOE_DTYPE_BF16, 1e-6f, &F, &F, &F, &F, nullptr,
+                                                   (const void*)0x2000, P, n, &w) == KMOE_OK);
+      if (route_mfma_fits(d, F)) {
+        const size_t KS = (size_t)route_mfma_splits(d), E = (size_t)l.E;
+        ok = ok && route_mfma_scratch_offsets(d, 2) - route_mfma_scratch_offsets(d, 1) >= 4 * KS * E &&
+             r - route_mfma_scratch_offsets(d, 2) >= 4 * KS * (size_t)T * E;
+      }
+    }
+    CHECK(ok);
+    // kmoe_route takes any scratch from the size of the transposed router and its norms
+    // on, whatever the tokens and the router
+    const kmoe_desc d = desc(4096, l.D, l.E, l.K, l.I, l.act, l.thr, l.impl == KMOE_IMPL_FIXED_CAPACITY ? 5 : 0, l.impl);
+    const size_t least = ((2 * (size_t)l.E * l.D + 255) & ~(size_t)255) + 4 * (((size_t)l.D + 255) / 256) * (size_t)l.E;
+    CHECK(route_scratch_min_bytes(d) == least && first_rs >= least);
+    const kmoe_weight* routers[] = {&F, &fr, &W};
+    for (const kmoe_weight* r : routers) {
+      EXPECT(validate_route(&d, P, r, P, least, I32, F32, I32), KMOE_OK, nullptr);
+      EXPECT(validate_route(&d, P, r, P, least - 1, I32, F32, I32), KMOE_ERR_WORKSPACE_TOO_SMALL, "scratch");
+    }
+    if (!route_mfma_fits(d, F)) CHECK(rs == least);
+  }
+}
+
 int main() {
   desc_cases();
   forward_cases();
@@ -378,6 +438,7 @@ int main() {
   block_cases();
   noalloc_cases();
   layout_sweep();
+  sizes_never_fall();
   CHECK(strcmp(status_string((kmoe_status)99), "unknown status") == 0);
   for (int s = 0; s < 6; ++s) CHECK(status_string((kmoe_status)s)[0] != '\0');
   if (g_fail) {

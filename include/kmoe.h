@@ -223,11 +223,12 @@ kmoe_status kmoe_rms_norm(const kmoe_desc* desc, const void* x, const void* scal
  * rounded to x.dtype, block_hist [ceil(T/64), E] int32 (per 64-token chunk
  * expert counts consumed by kmoe_dispatch). `scratch` (optional, may be NULL)
  * of kmoe_route_scratch_bytes(desc) bytes lets a call without logits take the
- * two-phase form when x and the router are bf16 and 16-byte aligned, D is a
- * multiple of 256 from 512 to 4096, E % 16 == 0 and E <= 256: every logit on the matrix cores, then the
- * canonical order only for the experts within a rigorous f32 error bound of the
- * K-th (the form kmoe_forward uses for most calls above 240 tokens). Selections, weights and
- * block_hist are the same either way. */
+ * two-phase form when x and the router are bf16, x, the router and the scratch are
+ * 16-byte aligned, D is a multiple of 256 from 512 to 4096, E % 16 == 0 and
+ * E <= 256: every logit on the matrix cores, then the canonical order only for the
+ * experts within a rigorous f32 error bound of the K-th (the form kmoe_forward
+ * uses for most calls above 240 tokens). Selections, weights and block_hist are the
+ * same either way. */
 kmoe_status kmoe_route(const kmoe_desc* desc, const void* x, const kmoe_weight* router, float* logits,
                        void* scratch, size_t scratch_bytes, int32_t* topk_idx, float* topk_w, int32_t* block_hist,
                        void* stream);

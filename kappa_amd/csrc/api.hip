@@ -89,7 +89,7 @@ kmoe_status kmoe_route(const kmoe_desc* desc, const void* x, const kmoe_weight* 
   if (desc->tokens == 0) return KMOE_OK;
   hipError_t e =
       !logits && scratch && route_mfma_fits(*desc, *router) && aligned16(x) && aligned16(router->values) &&
-              scratch_bytes >= route_mfma_scratch_bytes(*desc)
+              aligned16(scratch) && scratch_bytes >= route_mfma_scratch_bytes(*desc)
           ? launch_route_mfma(*desc, x, *router, scratch, topk_idx, topk_w, block_hist, (hipStream_t)stream)
           : launch_route(*desc, x, *router, logits, topk_idx, topk_w, block_hist, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "route kernels");
@@ -246,7 +246,7 @@ kmoe_status forward_general(const kmoe_desc* desc, const void* x, const void* xi
       KMOE_HIP(launch_rms_norm(*desc, x, norm->scale, norm->scale_bf16 ? KMOE_DTYPE_BF16 : KMOE_DTYPE_F32,
                                           norm->eps, norm->h2, st),
                "rms_norm kernel");
-    const int64_t scratch = route_mfma_place(*desc, xin, *router, w);
+    const int64_t scratch = aligned16(base) ? route_mfma_place(*desc, xin, *router, w) : -1;
     if (scratch >= 0)
       KMOE_HIP(launch_route_mfma(*desc, xin, *router, base + scratch, tidx, tw, hist, st), "route kernels");
     else

@@ -65,6 +65,64 @@ def test_route_off_alignment(dev):
         assert torch.equal(got[n], want[n]), n
 
 
+@pytest.mark.parametrize("short,shift", [(0, 0), (0, 4), (1, 0)])
+def test_route_scratch_forms(dev, short, shift):
+    """kmoe_route with its scratch, with one that is not 16-byte aligned, and with one
+    that is too small for the two-phase form: the selections of a call without."""
+    import ctypes
+
+    from kappa_amd import _lib
+    from kappa_amd.qwen3 import moe_stages
+    from kappa_amd.qwen3.ffn_moe import _desc, _stream
+    from kappa_amd.qwen3.quant import weight_struct
+
+    T, D, E, K = 300, 1024, 64, 4
+    g = torch.Generator(device="cuda").manual_seed(8)
+    x = torch.randn(T, D, generator=g, device=dev).to(torch.bfloat16)
+    router = (torch.randn(D, E, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    want = moe_stages.route(x, router, num_experts=E, k=K)
+    desc = _desc(T, D, E, K, 1, x.dtype)
+    r, keep = weight_struct(router, dev, n_out=E, n_groups=None, name="router_w")
+    n = ctypes.c_size_t()
+    _lib.check(_lib.lib().kmoe_route_scratch_bytes(desc, ctypes.byref(n)))
+    buf = torch.zeros(n.value + 64, dtype=torch.uint8, device=dev)
+    got = {k: torch.full_like(want[k], -1) for k in ("idx", "w", "hist")}
+    _lib.check(_lib.lib().kmoe_route(desc, x.data_ptr(), r, None, buf.data_ptr() + shift, n.value - short,
+                                     got["idx"].data_ptr(), got["w"].data_ptr(), got["hist"].data_ptr(), _stream(dev)))  # fmt: skip
+    for k in got:
+        assert torch.equal(got[k], want[k]), k
+    assert bool(buf.any()) == (not short and not shift)
+
+
+def test_workspace_off_alignment(dev):
+    """A workspace that is not 16-byte aligned (layout-native f32 weights, which ask for no
+    alignment of it): the output of an aligned one."""
+    import ctypes
+
+    from kappa_amd import _lib
+    from kappa_amd.qwen3.ffn_moe import _desc, _stream
+    from kappa_amd.qwen3.quant import weight_struct
+
+    T, D, E, K, I = 260, 512, 32, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn(T, D, generator=g, device=dev).to(torch.bfloat16)
+    router = (torch.randn(D, E, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    ws = [torch.randn(*s, generator=g, device=dev) * 0.05 for s in ((E, D, I), (E, D, I), (E, I, D))]
+    desc = _desc(T, D, E, K, I, x.dtype)
+    n = ctypes.c_size_t()
+    _lib.check(_lib.lib().kmoe_workspace_bytes(desc, ctypes.byref(n)))
+    buf = torch.zeros(n.value + 64, dtype=torch.uint8, device=dev)
+    args = [weight_struct(w, dev, n_out=w.shape[-1], n_groups=None if w is router else E, name="w")
+            for w in (router, *ws)]  # fmt: skip
+    outs = []
+    for shift in (0, 4):
+        out = torch.empty_like(x)
+        _lib.check(_lib.lib().kmoe_forward(desc, x.data_ptr(), *(a[0] for a in args), None, out.data_ptr(), None, None,
+                                           buf.data_ptr() + shift, n.value, _stream(dev)))  # fmt: skip
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("which", ["x", "scale"])
 def test_rms_norm_off_alignment(dev, dtype, which):

@@ -499,7 +499,9 @@ __global__ __launch_bounds__(256) void k_dispatch_scatter(int T, int E, int K, i
 // 2D roundings of up to 2u each, u = 2^-24), the canonical chains and tree (64 +
 // log2 P roundings), the rounding of the norms and of L~ -/+ delta (the host passes
 // c). So L lies in [lo, hi] = [L~ - delta, L~ + delta], delta = c * ||x_t|| * ||r_e|| +
-// 1e-30. Let tau be the K-th largest lo (the search stops at 16 key bits, which can
+// 1e-30. The norms are f32 sums of squares, each at least kNormFloor: below it squares
+// underflow and the computed sum says nothing, above it what underflow takes from
+// it (at most 4096 * 2^-126) is less than c's room. Let tau be the K-th largest lo (the search stops at 16 key bits, which can
 // only lower it). An expert whose hi is below tau has K experts strictly above
 // it and cannot be selected, ties included; the top K are among the
 // candidates {e : hi_e >= tau}. k_route_select recomputes the candidates' logits in
@@ -663,6 +665,7 @@ __device__ __forceinline__ uint32_t float_key(float v) {
   return (u >> 31) ? ~u : (u | 0x80000000u);
 }
 
+constexpr float kNormFloor = 0x1p-100f;  // of a squared norm
 constexpr int kSelectWaves = 4;        // tokens per block of k_route_select, one wave each
 constexpr int kRouteSliceBytes = 144;  // a 64-element bf16 slice of x in LDS, padded by 16 bytes
 
@@ -731,7 +734,7 @@ __global__ __launch_bounds__(64 * kSelectWaves, EPL <= 2 ? 4 : 2) void k_route_s
   }
 #pragma unroll
   for (int o = 1; o < P; o <<= 1) ss += __shfl_xor(ss, o, 64);
-  const float nxv = sqrtf(ss);
+  const float nxv = sqrtf(ss < kNormFloor ? kNormFloor : ss);
   float lo[EPL], hi[EPL];
   bool bad = !(nxv <= 3.0e38f);
 #pragma unroll
@@ -745,7 +748,7 @@ __global__ __launch_bounds__(64 * kSelectWaves, EPL <= 2 ? 4 : 2) void k_route_s
         v += pl[i][k];
         n2 += pn[i][k];
       }
-      const float dl = __builtin_fmaf(cbound * nxv, sqrtf(n2), 1e-30f);
+      const float dl = __builtin_fmaf(cbound * nxv, sqrtf(n2 < kNormFloor ? kNormFloor : n2), 1e-30f);
       lo[i] = v - dl;
       hi[i] = v + dl;
       bad = bad || !(lo[i] >= -3.0e38f && hi[i] <= 3.0e38f);

@@ -65,6 +65,27 @@ def test_route_off_alignment(dev):
         assert torch.equal(got[n], want[n]), n
 
 
+def test_route_underflowing_norms(dev):
+    """Router columns whose squares all underflow in f32, with a tie at the K-th place that
+    another sum order breaks: expert 9's terms at hidden indices 32..63 are each below
+    half an ulp of its running canonical sum and vanish, but summed by themselves
+    they lift the logit over a value with few bits. The lower index has to win."""
+    from kappa_amd.qwen3 import moe_stages
+
+    T, D, E = 300, 512, 16
+    r = np.zeros((D, E), np.float32)
+    r[0, [3, 9]] = 2.0**-77 * (1 + 2.0**-7)
+    r[1, [3, 9]] = -(2.0**-97)
+    r[32:64, 9] = 250 / 256 * 2.0**-101
+    x = np.full((T, D), 2.0**30, np.float32)
+    lg = oracle.router_logits(x, r)
+    assert (lg[:, 3] == lg[:, 9]).all() and (lg[:, 3] > 0).all() and (np.float32(r[0, 3]) ** 2 == 0)
+    xd, rd = (torch.from_numpy(a).to(dev).to(torch.bfloat16) for a in (x, r))
+    assert torch.equal(xd.float().cpu(), torch.from_numpy(x)) and torch.equal(rd.float().cpu(), torch.from_numpy(r))
+    got = moe_stages.route(xd, rd, num_experts=E, k=1, logits=False)
+    assert (got["idx"] == 3).all()
+
+
 @pytest.mark.parametrize("short,shift", [(0, 0), (0, 4), (1, 0)])
 def test_route_scratch_forms(dev, short, shift):
     """kmoe_route with its scratch, with one that is not 16-byte aligned, and with one

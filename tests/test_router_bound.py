@@ -1,10 +1,12 @@
 """The two-phase router's candidate rule (CPU).
 
-k_route_mfma (kappa_amd/csrc/route.hip) computes every logit on the matrix cores,
-L~ = L + eps with |eps| <= delta_e = c * ||x|| * ||r_e|| (+1e-30), takes tau = the
-K-th largest of lo = L~ - delta, keeps the candidates {e : hi_e = L~_e + delta_e >= tau},
-recomputes their canonical logits L and ranks them (value descending, ties to the
-lower expert index, as lax.top_k, kappa/qwen3/ffn_moe.py:51). The claim: whatever
+k_route_logits (kappa_amd/csrc/route.hip) computes every logit on the matrix cores,
+L~ = L + eps with |eps| <= delta_e = c * ||x|| * ||r_e|| (+1e-30), the squared norms
+taken as at least 2^-100 (their squares may underflow); k_route_select takes tau = the
+K-th largest of lo = L~ - delta, cut to the upper 16 bits of its key, keeps the
+candidates {e : hi_e = L~_e + delta_e >= tau}, recomputes their canonical logits L and
+ranks them (value descending, ties to the lower expert index, as lax.top_k,
+kappa/qwen3/ffn_moe.py:51). The claim: whatever
 eps within the bound, the first K of that ranking are the top K of L. This restates
 the rule in float32 numpy and checks it against a stable sort with planted exact
 ties and near ties at the K-th place and eps pushed to the edge of the bound in the
@@ -15,6 +17,9 @@ cases.
 from __future__ import annotations
 
 import numpy as np
+import pytest
+
+import oracle
 
 F32 = np.float32
 
@@ -31,7 +36,7 @@ def select(L: np.ndarray, L_approx: np.ndarray, delta: np.ndarray, K: int) -> np
     rank among the candidates' exact logits."""
     lo = (L_approx - delta).astype(F32)
     hi = (L_approx + delta).astype(F32)
-    thr = np.sort(key(lo))[::-1][K - 1]
+    thr = np.sort(key(lo))[::-1][K - 1] & np.uint32(0xFFFF0000)
     cand = np.nonzero(key(hi) >= thr)[0]
     assert len(cand) >= K
     # value descending, ties to the lower index (np.lexsort: last key is primary)
@@ -115,3 +120,40 @@ def test_half_the_bound_misses():
         got = select(L, adversarial(L, delta, K, 0.999), delta / 2, K)
         misses += not np.array_equal(got, reference_topk(L, K))
     assert misses > 100
+
+
+def _norm(sum_of_squares, floor=F32(2.0**-100)):
+    return np.sqrt(np.maximum(np.asarray(sum_of_squares, F32), floor))
+
+
+def _kernel_delta(x, R, floor=F32(2.0**-100)):
+    """The kernel's delta of one token: norms from f32 sums of f32 squares."""
+    D = len(x)
+    c = F32(np.ldexp(4.0 * D + 512.0, -24))
+    n2 = np.zeros(R.shape[1], F32)
+    for d in range(D):
+        n2 = n2 + R[d] * R[d]
+    return c * _norm(np.sum(x * x, dtype=F32), floor) * _norm(n2, floor) + F32(1e-30)
+
+
+@pytest.mark.parametrize("x_scale,r_scale", [(1.0, 0.02), (1.0, 2e-24), (1e8, 3e-24), (1e-24, 1.0), (1e-20, 1e-20)])
+def test_bound_covers_the_sum_order(x_scale, r_scale):
+    """|L~ - L| <= delta for f32 logits summed in the split order, also where every square
+    of the router or of the token underflows. Without the floor under the norms the
+    bound fails there."""
+    rng = np.random.default_rng(3)
+    D, E, T = 512, 32, 64
+    x = oracle.bf16_round((rng.standard_normal((T, D)) * x_scale).astype(F32))
+    R = oracle.bf16_round((rng.standard_normal((D, E)) * r_scale).astype(F32))
+    L = oracle.router_logits(x, R)
+    approx = np.zeros((T, E), F32)
+    for k in range(8):  # a split's sum, then the splits
+        part = np.zeros((T, E), F32)
+        for d in range(64 * k, 64 * k + 64):
+            part = part + (x[:, d : d + 1] * R[d]).astype(F32)
+        approx = approx + part
+    err = np.abs(approx.astype(np.float64) - L)
+    ratio = max(float((err[t] / _kernel_delta(x[t], R)).max()) for t in range(T))
+    assert ratio <= 1.0, ratio
+    if (x_scale, r_scale) == (1e8, 3e-24):
+        assert max(float((err[t] / _kernel_delta(x[t], R, F32(0))).max()) for t in range(T)) > 1.0

@@ -856,8 +856,11 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmLoads<GemmSha
   // 288 -> 281 and 457 -> 447 us, 235B-A22B T = 2048 808 -> 780 us. The priority
   // alone, or the prefetch without the fixed order, gained nothing; the static
   // priority of one block over the other lost 2%. The 64-row form (three blocks per
-  // CU, bound by the weight stream) is left to the compiler's order: held to this
-  // one, 30B-A3B T = 333 took 165 us instead of 163.
+  // CU, bound by the weight stream) issues its loads before it reads anything and is
+  // left to the compiler's order: held to this one, 30B-A3B T = 333 took 165 us instead
+  // of 163, and with the reads before the loads 30B-A3B T = 100 / 150 / 200 took 143.2 /
+  // 147.4 / 149.3 us instead of 140.8 / 145.6 / 146.9, 235B-A22B T = 150 434.6 instead of
+  // 431.4 (four interleaved rounds).
   constexpr bool kOrdered = RW > 64;
   constexpr int NK = 2 * MT;
   constexpr int PF = kOrdered ? (NK < 3 ? NK : 3) : 1;
@@ -866,18 +869,21 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmLoads<GemmSha
     const bool fresh = PL == 1 || (c & 1) == 0;  // a new weight chunk
     bool b_ahead = false;  // a weight chunk issued this iteration
     uint4 raw[4];
-    if (fresh) {
+    auto read_raw = [&]() {
       const uint8_t* bp = bring + (b % kGemmNB) * kGemmB + wv * 4096 + lane * 16;
 #pragma unroll
       for (int g = 0; g < 4; ++g) raw[g] = *reinterpret_cast<const uint4*>(bp + g * 1024);
-    }
+    };
     const uint16_t* As = reinterpret_cast<const uint16_t*>(smem + (c & 1) * kGemmA);
     auto a_read = [&](int k) {
       return *reinterpret_cast<const bf16x8*>(As + a_at<1>((k % MT) * 16 + (lane & 15), 2 * (lane >> 4) + k / MT));
     };
     bf16x8 af[PF];
+    if constexpr (kOrdered) {
+      if (fresh) read_raw();
 #pragma unroll
-    for (int k = 0; k < PF; ++k) af[k] = a_read(k);
+      for (int k = 0; k < PF; ++k) af[k] = a_read(k);
+    }
     if (c + 1 < KC) issue_a(c + 1);
     if (PL == 1 && c + kAhead < KC) {
       issue_b(c + kAhead);
@@ -888,17 +894,20 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmLoads<GemmSha
       b_ahead = true;
     }
     if (fresh) {
+      if constexpr (!kOrdered) read_raw();
 #pragma unroll
       for (int g = 0; g < 4; ++g) weights16<CH>(raw[g], gl.sc[g], lo[g], hi[g]);
     }
     if constexpr (kOrdered) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
+      if constexpr (!kOrdered) af[0] = a_read(k);
       // weights as the first operand: the accumulator tile is the output
       // transposed, so a lane holds four consecutive columns of one row
 #pragma unroll
       for (int g = 0; g < 4; ++g) acc[k % MT][g] = mfma16(k < MT ? lo[g] : hi[g], af[k % PF], acc[k % MT][g]);
-      if (k + PF < NK) af[k % PF] = a_read(k + PF);
+      if constexpr (kOrdered)
+        if (k + PF < NK) af[k % PF] = a_read(k + PF);
     }
     if constexpr (kOrdered) __builtin_amdgcn_s_setprio(0);
     // the order the compiler is held to (it otherwise reads a fragment right before its

@@ -73,21 +73,28 @@ bool route_mfma_preferred(const kmoe_desc& d, const kmoe_weight& router) {
   return route_mfma_fits(d, router) && d.tokens >= kRouteOwnScratchTokens;
 }
 
-// Just above 510 tokens the all-VALU router's blocks of two tokens fill the chip's CUs
-// once, and it beats the two-phase router's latency: whole layers, all-VALU against
-// two-phase, 30B-A3B T = 512 / 560 / 600 / 640 159 / 166 / 168.6 / 170.6 against 165 / 169 /
-// 169.7 / 169.7 us; D = 2560, E = 64, T = 512 / 576 / 640 154 / 162 / 170 against 159 / 165 /
-// 169; 235B-A22B T = 511 / 576 484 / 508 against 493 / 503; E = 256, T = 512 / 576 260 / 280
-// against 262 / 266. On either side (blocks of one token, or a second round) it is
-// 5 to 30 us behind, and so with 32 experts (T = 512 127 against 117).
-static bool route_one_round(const kmoe_desc& d) {
-  const int64_t blocks = (d.tokens + 1) / 2;
-  const int64_t most = d.hidden <= 2560 && d.num_experts <= 128 ? 300 : 256;
-  return d.num_experts >= 64 && blocks >= 256 && blocks <= most;
+// The sizes above the split router's at which the all-VALU router is the faster one.
+// Its blocks take one token up to 510, two up to 1020, and each reads the whole router,
+// so its time steps with the blocks per CU; the two-phase router's hardly depends on T,
+// but above D = 2048 its canonical chains take 64 lanes instead of 32, 7 us more.
+// Whole layers in one process, all-VALU less two-phase in us:
+//   one block per CU: D = 2304 .. 4096, T = 241 / 256 with 32 to 256 experts -9 .. +1 (16:
+//     0 .. +3); D <= 2048 there 0 .. +9. T = 511 / 512 with a router of 256 KB or more -11 .. 0;
+//     smaller ones (1024 x 64 and 96, 512 x 64) 0 .. +5, 16 experts +5 .. +20.
+//   D = 2304 .. 3072 with 32 to 64 experts, whose 8-wave blocks share a CU: T = 257 .. 1020
+//     -7 .. 0 (4096 x 64 at T = 257 .. 510 0 .. +4; from 1021 on 0 .. +10).
+//   else: 30B-A3B T = 257 .. 510 +9, 520 .. 1020 0 .. +1, 1100 +10; 235B-A22B +21, +9, +28; D = 2048,
+//     E = 256 +32, +14, +26; D = 2560, E = 80 .. 128 +11, +5, +20; 32 experts at D <= 2048 +2 .. +18.
+static bool route_all_valu(const kmoe_desc& d) {
+  const int64_t T = d.tokens, D = d.hidden, E = d.num_experts;
+  if (E < 32) return false;
+  if (T <= 256) return D > 2048;
+  if (T == 511 || T == 512) return D * E >= 131072;
+  return T <= 1020 && D > 2048 && D <= 3072 && E <= 64;
 }
 
 int64_t route_mfma_place(const kmoe_desc& d, const void* x, const kmoe_weight& router, const Workspace& w) {
-  if (!route_mfma_fits(d, router) || !aligned16(x) || !aligned16(router.values) || route_one_round(d)) return -1;
+  if (!route_mfma_fits(d, router) || !aligned16(x) || !aligned16(router.values) || route_all_valu(d)) return -1;
   if (route_mfma_preferred(d, router)) return (int64_t)w.route_part;
   return w.route_part - w.h_sorted >= route_mfma_scratch_bytes(d) ? (int64_t)w.h_sorted : -1;
 }

@@ -169,7 +169,7 @@ Workspace layout(const kmoe_desc& d, bool block);
 // Workspace offset of the two-phase router's scratch for this call; -1 where the
 // all-VALU router runs instead (the shape does not fit, x or the router is not
 // 16-byte aligned, h_sorted and y_sorted are smaller than the scratch, or it is the
-// faster one: just above 510 tokens).
+// faster one).
 int64_t route_mfma_place(const kmoe_desc& d, const void* x, const kmoe_weight& router, const Workspace& w);
 
 // --- argument checks ---------------------------------------------------------

@@ -371,6 +371,49 @@ static void layout_sweep() {
             }
 }
 
+// Which router a whole call above the split router's sizes takes: at the edges of the
+// sizes that the all-VALU one keeps, and where the two-phase one cannot run.
+static void router_choice() {
+  const kmoe_weight fr = weight(P, KMOE_DTYPE_F32, nullptr, KMOE_DTYPE_F32, KMOE_SCALE_NONE);
+  const kmoe_weight off = weight(reinterpret_cast<const void*>(0x1002), KMOE_DTYPE_BF16, nullptr, KMOE_DTYPE_F32,
+                                 KMOE_SCALE_NONE);
+  auto two_phase = [](const kmoe_desc& d, const kmoe_weight& r, const void* x) {
+    const Workspace w = layout(d, false);
+    const int64_t at = route_mfma_place(d, x, r, w);
+    if (at < 0) return false;
+    // inside its buffers, and what it holds there fits
+    const size_t end = d.tokens >= kRouteOwnScratchTokens ? w.h_scale : w.route_part;
+    CHECK((size_t)at == (d.tokens >= kRouteOwnScratchTokens ? w.route_part : w.h_sorted) &&
+          (size_t)at + route_mfma_scratch_bytes(d) <= end);
+    return true;
+  };
+  struct {
+    int64_t D, E, K, I, T;
+    bool two;
+  } cases[] = {
+      // 30B-A3B: the two-token blocks that come one per CU
+      {2048, 128, 8, 768, 241, true}, {2048, 128, 8, 768, 510, true}, {2048, 128, 8, 768, 511, false},
+      {2048, 128, 8, 768, 512, false}, {2048, 128, 8, 768, 513, true}, {2048, 128, 8, 768, 600, true},
+      {2048, 128, 8, 768, 2047, true}, {2048, 128, 8, 768, 2048, true}, {2048, 128, 8, 768, 4096, true},
+      // rows above 2048: also the one-token blocks
+      {4096, 128, 8, 1536, 256, false}, {4096, 128, 8, 1536, 257, true}, {4096, 128, 8, 1536, 512, false},
+      {4096, 128, 8, 1536, 513, true},
+      // and few experts up to the two-token blocks' last size
+      {2560, 64, 6, 1024, 241, false}, {2560, 64, 6, 1024, 300, false}, {2560, 64, 6, 1024, 1020, false},
+      {2560, 64, 6, 1024, 1021, true}, {2560, 80, 6, 1024, 300, true}, {3328, 64, 6, 1024, 300, true},
+      {2560, 16, 4, 1024, 256, true}, {2560, 16, 4, 1024, 512, true},
+      // a small router
+      {1024, 96, 8, 768, 512, true}, {1024, 128, 8, 768, 512, false},
+      // expert buffers smaller than the scratch
+      {512, 256, 1, 64, 300, false},
+  };
+  for (auto& c : cases) {
+    const kmoe_desc d = desc(c.T, c.D, c.E, c.K, c.I);
+    CHECK(two_phase(d, F, P) == c.two);
+    CHECK(!two_phase(d, fr, P) && !two_phase(d, off, P) && !two_phase(d, F, off.values));
+  }
+}
+
 // A caller sizes its buffers once, for its largest call: the reported sizes never
 // fall as the tokens grow, and every smaller call is accepted with them.
 static void sizes_never_fall() {
@@ -439,6 +482,7 @@ int main() {
   noalloc_cases();
   layout_sweep();
   sizes_never_fall();
+  router_choice();
   CHECK(strcmp(status_string((kmoe_status)99), "unknown status") == 0);
   for (int s = 0; s < 6; ++s) CHECK(status_string((kmoe_status)s)[0] != '\0');
   if (g_fail) {

@@ -1,5 +1,7 @@
-"""Which router the layer call takes above 240 tokens, and rows that the norm takes
-element by element (GPU). Routing is compared bit for bit with the oracle."""
+"""Routing of the layer call above 240 tokens where the choice between its two routers
+changes (the choice itself is checked on the CPU, sanitize/host_checks.cpp), and rows
+that the norm takes element by element (GPU). Routing is compared bit for bit with the
+oracle."""
 
 from __future__ import annotations
 
@@ -23,11 +25,14 @@ def dev():
 # the first size of the two-phase router, with its scratch in the expert buffers; a
 # reduction of forty slices; expert buffers smaller than the scratch and a hidden size
 # it does not take (the all-VALU router); two halves of 128 experts, the second partial;
-# the edges of the sizes just above 510 tokens that the all-VALU router keeps
+# a small router at 511 tokens and one above; the sizes that the all-VALU router keeps,
+# and the first after them
 @pytest.mark.parametrize(
     "T,D,E,K,I",
     [(241, 512, 32, 4, 128), (300, 2560, 64, 6, 64), (300, 512, 256, 1, 64), (260, 640, 32, 2, 64),
-     (500, 768, 176, 8, 64), (511, 512, 64, 4, 64), (601, 512, 64, 4, 64)],
+     (500, 768, 176, 8, 64), (511, 512, 64, 4, 64), (601, 512, 64, 4, 64), (512, 2048, 64, 4, 64),
+     (513, 2048, 64, 4, 64), (256, 2304, 96, 4, 64), (257, 2304, 96, 4, 64), (1020, 2304, 48, 4, 64),
+     (1021, 2304, 48, 4, 64)],
 )  # fmt: skip
 def test_layer_routing_above_the_split_router(dev, T, D, E, K, I):
     from kappa_amd.qwen3 import quantize_weight

@@ -747,8 +747,8 @@ __global__ __launch_bounds__(256, 2) void k_prefill(int D, int I, int E, const u
 // itself (vmcnt is in-order), then a barrier publishes the stage and frees
 // the ones read last.
 //
-// Rows past the expert's end are loaded from a clamped copy of row 0 (up to the
-// next multiple of 16) and never stored; the loop body is instantiated for 1 to 8
+// Rows past the expert's end are loaded from a clamped copy of row 0 (in the larger
+// tiles up to the next multiple of 16) and never stored; the loop body is instantiated for 1 to 8
 // (10) active 16-row tiles.
 // Work items are ordered (expert, column tile, row tile) and consecutive items
 // go to the same XCD, so the row tiles of one expert share
@@ -808,8 +808,10 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmLoads<GemmSha
 #pragma unroll
     for (int g = 0; g < 4; ++g) acc[mi][g] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // rows past the tile's last 16-row block are not loaded
-  auto a_on = [&](int j) { return 32 * j + 8 * wv < 16 * MT; };
+  // rows past the tile's last 16-row block are not loaded; but the 64-row form, whose
+  // waves would then issue unequal loads, is no faster for it: 30B-A3B T = 150 / 333 /
+  // 512 144.4 / 156.7 / 158.3 us with every row, 144.5 / 157.1 / 159.4 without
+  auto a_on = [&](int j) { return RW == 64 || 32 * j + 8 * wv < 16 * MT; };
   auto issue_a = [&](int c) {
     const uint32_t st = lds0 + (uint32_t)((c & 1) * kGemmA + wv * 1024);
     const uint16_t* abase = src + (PL == 2 ? (c & 1) * (KCW * 64) + (c >> 1) * 64 : c * 64);

@@ -74,8 +74,21 @@ __global__ __launch_bounds__(256) void k_rms_norm(int T, int D, float eps, const
     }
     return;
   }
-  for (int d = lane; d < D; d += 64)
-    Act<A>::store(dst, d, rms_apply<A>(Act<A>::load(row, R::at(d)), r, Act<S>::load(scale, d)));
+  if constexpr (sizeof(A) == 2) {
+    for (int d = lane; d < D; d += 64)
+      Act<A>::store(dst, d, rms_apply<A>(Act<A>::load(row, R::at(d)), r, Act<S>::load(scale, d)));
+    return;
+  }
+  for (int base = 0; base < D; base += 64 * R::kBatch) {
+    float sc[R::kBatch];
+#pragma unroll
+    for (int j = 0; j < R::kBatch; ++j) sc[j] = Act<S>::load(scale, min(base + 64 * j + lane, D - 1));
+#pragma unroll
+    for (int j = 0; j < R::kBatch; ++j) {
+      const int d = base + 64 * j + lane;
+      if (d < D) Act<A>::store(dst, d, rms_apply<A>(Act<A>::load(row, R::at(d)), r, sc[j]));
+    }
+  }
 }
 
 }  // namespace kmoe

@@ -49,6 +49,18 @@ __device__ __forceinline__ u32x2 load_stream8(const char* base, uint32_t off) {
 
 constexpr int kW16Waves = 8;  // waves of a decode block, splitting the reduction
 
+// One output of the f32 chain's down product as the layout-native kernel sums it: h =
+// hi + lo first, then one chain. The planes meet a weight separately, so an infinite
+// weight gives inf - inf (or 0 * inf) where h * inf is infinite: outputs that come out
+// NaN are summed again this way. h: a row's hi plane (lo I further), w: the column.
+__device__ __forceinline__ float w16_chain(const uint16_t* __restrict__ h, int I, const uint16_t* __restrict__ w,
+                                           int D) {
+  float acc = 0.0f;
+  for (int i = 0; i < I; ++i)
+    acc = __builtin_fmaf(bf16_bits_to_f32(h[i]) + bf16_bits_to_f32(h[I + i]), bf16_bits_to_f32(w[(size_t)i * D]), acc);
+  return acc;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -209,7 +221,11 @@ __global__ __launch_bounds__(64 * kW16Waves, 4) void k_down_w16(int D, int I, in
   for (int w = 1; w < kW16Waves; ++w) v += red[w][wv][lane];
   uint16_t* yr = y_sorted + (size_t)(r0 + c) * D + col0 + 16 * q + wv;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) yr[4 * i] = f32_to_bf16_bits(v[i]);
+  for (int i = 0; i < 4; ++i) {
+    if (CH == kChainF32 && v[i] != v[i])
+      v[i] = w16_chain(h_sorted + (size_t)(r0 + c) * 2 * I, I, wd + (size_t)e * I * D + col0 + 16 * q + wv + 4 * i, D);
+    yr[4 * i] = f32_to_bf16_bits(v[i]);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -335,6 +351,8 @@ __device__ __forceinline__ void w16_tile(uint8_t* smem, const W16Loads& gl, int 
     }
   }
 
+  bool nan = false;  // of this lane's outputs (the f32 chain's down product)
+
   // a lane holds row mi * 16 + lane % 16 and, for i, g: gate/up columns 2 (4 q + i)
   // + g (up in tiles 2, 3), down columns 4 (4 q + i) + g, of the wave's columns
   if (!col_on) return;
@@ -375,6 +393,22 @@ __device__ __forceinline__ void w16_tile(uint8_t* smem, const W16Loads& gl, int 
         }
         *reinterpret_cast<uint4*>(drow + 8 * hf) = uint4{o[0], o[1], o[2], o[3]};
       }
+      if (CH == kChainF32) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) nan = nan || acc[mi][g][i] != acc[mi][g][i];
+      }
+    }
+  }
+  if (!GATEUP && CH == kChainF32 && nan) {
+    // summed again in the chain's order (w16_chain), from what was stored
+    for (int row = lane & 15; row < rows; row += 16) {
+      uint16_t* y = dst + (size_t)(row0 + row) * Ndim + col + 16 * (lane >> 4);
+      for (int j = 0; j < 16; ++j)
+        if ((y[j] & 0x7fffu) > 0x7f80u)
+          y[j] = f32_to_bf16_bits(w16_chain(src + (size_t)(row0 + row) * PL * KCW * 64, KCW * 64,
+                                            reinterpret_cast<const uint16_t*>(gl.b0) + 16 * (lane >> 4) + j, Ndim));
     }
   }
 }

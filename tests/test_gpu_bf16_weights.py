@@ -104,3 +104,21 @@ def test_bf16_stage_writes_every_row(dev, T):
                                impl="fixed_capacity")  # fmt: skip
     got = y.float().cpu().numpy()
     assert np.abs(got - ref).max() <= 2e-2 and mean_rel(got, ref) <= 1e-3
+
+
+@pytest.mark.parametrize("impl", ["gather_einsum", "ragged"])
+@pytest.mark.parametrize("T", [5, 100])
+def test_bf16_infinite_weight(dev, T, impl):
+    """An infinite down weight gives the infinities of the chain's order, not NaN where h's
+    two planes differ in sign or the lower one is zero."""
+    xn, rn, *wn = _layer(T + 2, T)
+    wn[2][:, 5, 7] = np.inf
+    wn[2][1, 6, 9] = np.nan
+    ref = oracle.forward(xn, rn, *wn, k=K, act_bf16=True, impl=impl)
+    x, router, *ws = (_dev_bf16(a, dev) for a in (xn, rn, *wn))
+    out, _, _ = _forward(dev, x, router, ws, impl)
+    got = out.reshape(T, D).float().cpu().numpy()
+    fin = np.isfinite(ref["out"])
+    assert np.isinf(ref["out"][:, 7]).any() and np.isnan(ref["out"][:, 9]).any()
+    np.testing.assert_array_equal(got[~fin], ref["out"][~fin])
+    assert np.isfinite(got[fin]).all() and mean_rel(got[fin], ref["out"][fin]) <= 1e-3

@@ -52,8 +52,9 @@ def test_quantiser_edges(dev, rows, cols, dtype):
 
 @pytest.mark.parametrize("rows", [300, 2300])
 def test_quantiser_non_finite(dev, rows):
-    """Infinities and NaN quantise as one value divided at a time does (the kernel that
-    takes any alignment)."""
+    """Infinities and NaN against the oracle: NaN does not count for a channel's scale, and
+    a quotient that is NaN (which the oracle leaves to C's conversion) quantises to
+    -128. Both kernels: aligned, and of any alignment."""
     from kappa_amd.qwen3 import quantize_weight_per_channel
 
     g = torch.Generator(device=dev)
@@ -62,10 +63,15 @@ def test_quantiser_non_finite(dev, rows):
     w[0, 5, 0], w[0, 7, 1], w[0, rows - 1, 2], w[0, rows - 2, 3] = float("nan"), float("inf"), float("-inf"), 3e38
     w[0, :, 4] = float("nan")
     w[0, :, 5] *= 1e-37
-    q, s = quantize_weight_per_channel(w)
-    q2, s2 = quantize_weight_per_channel(_shifted(w))
-    assert torch.equal(q, q2)
-    assert torch.equal(s.view(torch.int32), s2.view(torch.int32))
+    wn = w.float().cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        qo, so = oracle.quantize_per_channel(wn)
+        nan = np.isnan(wn / so)
+    assert nan.any() and not nan.all()
+    for t in (w, _shifted(w)):
+        q, s = quantize_weight_per_channel(t)
+        np.testing.assert_array_equal(s.cpu().numpy().view(np.int32), so.view(np.int32))
+        np.testing.assert_array_equal(q.cpu().numpy(), np.where(nan, -128, qo))
 
 
 @pytest.mark.parametrize("E,D,I", [(2, 64, 64), (3, 320, 192), (1, 576, 1088)])

@@ -81,7 +81,9 @@ typedef enum kmoe_impl {
 
 /* Kernel family of the expert products. Every family follows the impl's rounding
  * points; they add the same products in different f32 orders, so results agree to
- * rounding but are not bit-identical across families. */
+ * rounding but are not bit-identical across families. Plain bf16 experts run on
+ * them too, where D and I are multiples of 64 and the buffers 16-byte aligned; else, as
+ * f32 and unpacked int8 experts, on the layout-native kernels (a third order). */
 typedef enum kmoe_kernels {
   KMOE_KERNELS_AUTO = 0,     /* by token count: GEMV-style up to 64 tokens, grouped GEMMs above */
   KMOE_KERNELS_DECODE = 1,   /* the GEMV-style kernels (at most 128 tokens; row groups above 64) */

@@ -18,7 +18,7 @@
 // The layout-native kernels (one fmaf chain per output, every assignment
 // reading its expert's weights again) took, for gate/up + down of the 30B-A3B
 // layer, 1045 + 314 us at T = 4 (gather) and 21.4 + 10.9 ms at T = 1024 (ragged);
-// these take 38 + 17 and 189 + 103 us.
+// these take 40 + 18 and 196 + 110 us.
 #include "common.h"
 #include "expert_dev.h"
 #include "launch.h"

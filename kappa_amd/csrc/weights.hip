@@ -31,7 +31,7 @@ __device__ __forceinline__ void transpose4x4(const uint32_t* r, uint32_t* c) {
 // reads 256 consecutive bytes of each row, all 16 rows in flight) and four 16-byte
 // stores, 64 consecutive bytes; the waves of a block take consecutive k groups,
 // whose cells are consecutive. Bound by HBM: 30B-A3B gate + up + down (1.2 GB moved)
-// 235-255 us (4.7-5.1 TB/s). One 16-byte cell per thread from 16 byte loads took
+// 235-260 us (4.6-5.1 TB/s). One 16-byte cell per thread from 16 byte loads took
 // 516 us.
 // Source rows need no alignment.
 __global__ __launch_bounds__(256) void k_pack(int Kd, int N, int W, const int8_t* __restrict__ src0,

@@ -201,7 +201,7 @@ static void stage_cases() {
   CHECK(rs >= (size_t)2 * 8 * 128 + 4 * 8);  // the bf16 transposed router and the norm partials
   EXPECT(validate_route(&d, P, &F, P, rs - 1, I, Fp, I), KMOE_ERR_WORKSPACE_TOO_SMALL, "scratch");
   EXPECT(validate_route(&d, P, &F, P, rs, I, Fp, I), KMOE_OK, nullptr);
-  // the two-phase form's shapes: bf16 activations and router, 512 <= D <= 4096, D % 64, E % 16
+  // the two-phase form's shapes: bf16 activations and router, 512 <= D <= 4096, D % 256, E % 16
   const kmoe_weight RB = weight(P, KMOE_DTYPE_BF16, nullptr, KMOE_DTYPE_F32, KMOE_SCALE_NONE);
   const kmoe_desc l30 = desc(4096, 2048, 128, 8, 768);
   CHECK(route_mfma_fits(l30, RB) && !route_mfma_fits(l30, W) && !route_mfma_fits(desc(4096, 256, 128, 8), RB));

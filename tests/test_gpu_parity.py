@@ -982,9 +982,9 @@ def test_two_phase_router_ties_near_ties_and_fallback(dev):
 
 @pytest.mark.parametrize("T", [512, 2048, 2049, 3001, 4096])
 def test_forward_routing_two_phase(dev, l30, T):
-    """kmoe_forward from 2048 tokens routes with the two-phase form (below, the
-    all-VALU router): its indices and weights equal the stage router's, also
-    where its last block holds fewer than 16 tokens (T = 2049, 3001)."""
+    """kmoe_forward routes with the two-phase form from 2048 tokens (and at most
+    smaller sizes above 240; not at 512): its indices and weights equal the stage
+    router's, also where its last block is nearly empty (T = 2049, 3001)."""
     from kappa_amd.qwen3 import moe_stages
     from kappa_amd.qwen3.ffn_moe import _moe_forward
 
